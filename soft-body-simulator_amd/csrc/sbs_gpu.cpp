@@ -21,6 +21,7 @@
 #include "body_contact.h"
 #include "contact_hash.h"
 #include "grid_sdf.h"
+#include "island.h"
 #include "kernels.h"
 #include "scan_sort.h"
 #include "mlp.h"
@@ -77,6 +78,11 @@ struct group_t {
     // use, 0, 0, 0)
     dev_buf<uint4> ws_cinfo;
     uint32_t ws_rows = 0;
+    // small bodies: inside each color the elements run body by body, and per body and color
+    // (first element, first constraint, constraint stride of a cluster's tets, elements); empty
+    // when the group runs one launch per color
+    std::vector<uint4> body_stages;
+    uint32_t largest_stage = 0;
     std::vector<uint32_t> ws_rowof;  // cluster -> its row
     bool clustered() const { return !cluster_off.empty(); }
     uint32_t body_of(uint32_t c) const { return cbody.empty() ? body : cbody[c]; }
@@ -168,6 +174,14 @@ struct sbs_gpu {
                 bnbr.p, bvt_off.p, bvt.p, btn.p, bsph.p, btlo.p, btpx.p, berec.p, besph.p, bvn.p};
     }
     void setup_body_contacts(std::vector<uint4> const& tr, std::vector<pos4> const& x);
+
+    // whole-frame launches (island.hip): one workgroup per body; no rows when the scene has none
+    dev_buf<uint4> islands, island_stages;
+    dev_buf<uint32_t> island_list;
+    uint32_t island_largest = 0;
+    void plan_islands();
+    bool runs_islands() const { return islands.n && !timing && !(cap_net && cap_stride); }
+    void launch_islands(double dt, uint32_t iterations, uint32_t substeps, bool whole, bool warmed, bool contacts_done);
 
     int block = 256;
     int cluster_block = 64;
@@ -318,6 +332,7 @@ struct sbs_gpu {
 
     void commit(uint32_t recolor_passes);
     void color_group(group_t& g, uint32_t recolor_passes);
+    bool small_bodies(group_t const& g) const;
     void upload_group(group_t& g);
     void enqueue_frame(double dt, uint32_t iterations, uint32_t substeps, int warm, bool check = false);
     void run_frame(double dt, uint32_t iterations, uint32_t substeps, int warm, bool check = false);
@@ -451,6 +466,45 @@ void sbs_gpu::color_group(group_t& g, uint32_t recolor_passes)
     }
 }
 
+// Whether the scene's frames run one workgroup per body (island.hip) instead of one launch per color:
+// every body's particles fit LDS, and the estimated time of a stage (one color of every body) is shorter.
+// A launch takes 5.1 us and 0.16 us per 1,000 hex cells (5.4 us at 2,700 cells a color, 8.2 at 20,800, 17
+// at 83,000, 82 at 445,000); a body's stage takes 3.5-4.3 us up to 256 cells (3.50 at 64, 3.82 at 128, 4.25
+// at 256), 5.4-5.8 up to 512, 7.6 up to 640, and the bodies share 256 compute units. Measured: 24x6x6 cells
+// 6.2 us a stage launched, 3.7 here; one body of 512 cells a color 5.1 launched, 5.8 here; 512 bodies of 2,900
+// to 6,500 tets 12.3 and 5.6; 512 bodies of 8,000 to 14,000 tets 26.9 and 9.9. Green cells: 13.5-16 us
+// launched; 11.6-12.5 here up to 256 cells, 16.5 at 512. Single tets: 2.1-4.9 us launched, 1.05-1.9
+// (neo-Hookean) and 2.4-4.6 (Green) here at any size that fits LDS.
+bool sbs_gpu::small_bodies(group_t const& g) const
+{
+    if (g.kind == 2 || body_contacts || g.count >= kIslandConstraints) return false;
+    for (auto const& o : groups)
+        if (&o != &g && o.count) return false;
+    for (auto const& b : bodies)
+        if (b.n > kIslandParticles) return false;
+    uint32_t const ne = g.num_elements();
+    std::vector<uint32_t> counts(bodies.size() * std::size_t(g.ncolors), 0);
+    for (uint32_t e = 0; e < ne; ++e) {
+        uint32_t const c0 = g.clustered() ? g.cluster_off[e] : e, c1 = g.clustered() ? g.cluster_off[e + 1] : e + 1;
+        uint32_t const b = g.body_of(c0);
+        for (uint32_t c = c0 + 1; c < c1; ++c)
+            if (g.body_of(c) != b) return false;  // a cluster over two bodies
+        ++counts[std::size_t(b) * g.ncolors + g.color[c0]];
+    }
+    if (!g.clustered()) return true;
+    double longest = 0.0, sum = 0.0;
+    for (std::size_t b = 0; b < bodies.size(); ++b) {
+        uint32_t n = 0;
+        for (uint32_t c = 0; c < g.ncolors; ++c) n = std::max(n, counts[b * g.ncolors + c]);
+        double const green = 11.5 + 0.0025 * n + (n > 256 ? 3.5 : 0.0);
+        double const nh = n <= 256 ? 3.4 + 0.0033 * n : 3.4 + 0.0033 * 256 + 1.8 * ((n - 1) / 256);
+        longest = std::max(longest, g.kind == 0 ? green : nh);
+        sum += g.kind == 0 ? green : nh;
+    }
+    double const per_color = double(ne) / std::max<uint32_t>(g.ncolors, 1);
+    return std::max(longest, sum / 256.0) < (g.kind == 0 ? 13.5 + 0.18e-3 * per_color : 5.1 + 0.16e-3 * per_color);
+}
+
 // Lays a group out in color order (stable by insertion index) and uploads it in FP32; the rest
 // shape inverse and volume are computed in FP64 first (green_constraint.cpp:38-46).
 void sbs_gpu::upload_group(group_t& g)
@@ -476,7 +530,21 @@ void sbs_gpu::upload_group(group_t& g)
         std::vector<uint32_t> fill(g.cluster_color_offsets.begin(), g.cluster_color_offsets.end() - 1);
         for (uint32_t e = 0; e < ne; ++e) eorder[fill[g.color[e_begin(e)]]++] = e;
     }
-    if (g.clustered()) {
+    bool const by_body = small_bodies(g);
+    if (by_body) {
+        // body by body inside each color (a body's elements are then one run of it); elements of
+        // one color are independent, so their order does not change the result
+        for (uint32_t c = 0; c < g.ncolors; ++c)
+            std::stable_sort(eorder.begin() + g.cluster_color_offsets[c], eorder.begin() + g.cluster_color_offsets[c + 1],
+                             [&](uint32_t a, uint32_t b) { return g.body_of(e_begin(a)) < g.body_of(e_begin(b)); });
+        if (g.clustered()) {
+            g.xsplit.assign(g.ncolors, xcd_split{});
+            for (uint32_t c = 0; c < g.ncolors; ++c) {
+                uint64_t const n = g.cluster_color_offsets[c + 1] - g.cluster_color_offsets[c];
+                for (int x = 0; x <= kXcds; ++x) g.xsplit[c].off[x] = uint32_t(n * uint32_t(x) / kXcds);
+            }
+        }
+    } else if (g.clustered()) {
         // XCD affinity: the clusters in Morton order of their first constraint's rest centroid,
         // split into 8 regions of equal count; inside each color, clusters by region, then by
         // index (the caller's order, which keeps neighbouring clusters' particle gathers
@@ -585,6 +653,21 @@ void sbs_gpu::upload_group(group_t& g)
         g.cl_loc.upload(loc.data(), loc.size(), stream);
         g.cl_v0.upload(v0.data(), v0.size(), stream);
         g.cl_v1.upload(v1.data(), v1.size(), stream);
+    }
+    g.body_stages.clear();
+    g.largest_stage = 0;
+    if (by_body && (g.hex || !g.clustered())) {
+        g.body_stages.assign(bodies.size() * g.ncolors, make_uint4(0, 0, 0, 0));
+        for (uint32_t c = 0; c < g.ncolors; ++c) {
+            uint32_t const cb = g.cluster_color_offsets[c], ce = g.cluster_color_offsets[c + 1];
+            for (uint32_t j = cb; j < ce;) {
+                uint32_t const b = g.body_of(e_begin(eorder[j])), first = j;
+                while (j < ce && g.body_of(e_begin(eorder[j])) == b) ++j;
+                g.body_stages[std::size_t(b) * g.ncolors + c] =
+                    make_uint4(first, g.color_offsets[c] + (first - cb), ce - cb, j - first);
+                g.largest_stage = std::max(g.largest_stage, j - first);
+            }
+        }
     }
     if (g.kind == 2) {
         std::vector<uint2> idx(n);
@@ -759,8 +842,69 @@ void sbs_gpu::commit(uint32_t recolor_passes)
         build_hash();
         if (bodies_collide) setup_body_contacts(tr, x);
     }
+    plan_islands();
     hip_check(hipStreamSynchronize(stream), "commit");
     committed = true;
+}
+
+// The bodies as islands (small_bodies decided so when their group was laid out).
+void sbs_gpu::plan_islands()
+{
+    group_t const* g = nullptr;
+    for (auto const& o : groups)
+        if (o.count) g = &o;
+    if (!g || g->body_stages.empty()) return;
+    std::vector<uint4> rec;
+    std::vector<uint64_t> work(bodies.size(), 0);
+    uint32_t base = 0;
+    for (std::size_t b = 0; b < bodies.size(); ++b) {
+        rec.push_back(make_uint4(bodies[b].offset, bodies[b].n, base, uint32_t(bodies[b].surface.size())));
+        base += uint32_t(bodies[b].surface.size());
+        island_largest = std::max(island_largest, bodies[b].n);
+        for (uint32_t c = 0; c < g->ncolors; ++c) work[b] += g->body_stages[b * g->ncolors + c].w;
+    }
+    // the longest first: workgroups start in order, and the last ones to end should be short
+    std::vector<uint32_t> order(bodies.size());
+    std::iota(order.begin(), order.end(), 0u);
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return work[a] > work[b]; });
+    std::vector<uint4> sorted, stages;
+    for (uint32_t b : order) {
+        sorted.push_back(rec[b]);
+        stages.insert(stages.end(), g->body_stages.begin() + std::size_t(b) * g->ncolors,
+                      g->body_stages.begin() + (std::size_t(b) + 1) * g->ncolors);
+    }
+    islands.upload(sorted.data(), sorted.size(), stream);
+    island_stages.upload(stages.data(), stages.size(), stream);
+    island_list.alloc(std::max<uint32_t>(S, 1));
+    hip_check(hipStreamSynchronize(stream), "upload islands");
+}
+
+// The whole frame of every body in one launch, or (whole false) one substep's iterations between its
+// prediction and its velocity update.
+void sbs_gpu::launch_islands(double dt, uint32_t iterations, uint32_t substeps, bool whole, bool warmed,
+                             bool contacts_done)
+{
+    group_t const* g = nullptr;
+    for (auto const& o : groups)
+        if (o.count) g = &o;
+    double const dt2 = dt * dt, at = g->alpha / dt2;
+    solve_params p{};
+    p.substeps = substeps;
+    p.iterations = iterations;
+    p.predict = p.commit = whole;
+    p.zero_first = !warmed;
+    p.skip_first_contacts = contacts_done;
+    p.dt = float(dt);
+    for (int d = 0; d < 3; ++d) p.g[d] = float(params.gravity[d]);
+    p.force = params.gravity_is_force;
+    p.contact_at = float(params.collision_compliance / dt2);
+    p.alpha_tilde = float(at);
+    p.gamma = float(at * (g->beta * dt2) / dt);
+    p.inv_dt2 = float(1.0 / dt2);
+    p.beta_dt = float(g->beta * dt);
+    island_dev const d{islands.p, island_stages.p, island_list.p, uint32_t(islands.n), g->ncolors,
+                       island_largest, g->largest_stage};
+    launch_island_frame(stream, d, g->kind, g->hex, g->tet(), g->clusters(), xi.p, xn.p, vel.p, contacts(), p);
 }
 
 void sbs_gpu::detect()
@@ -997,7 +1141,10 @@ void sbs_gpu::enqueue_frame(double dt_frame, uint32_t iterations, uint32_t subst
     contact_dev const c = contacts();
     float const c_at = float(params.collision_compliance / dt2);
     bool const capture = cap_net != nullptr && cap_stride > 0;
-    for (uint32_t s = 0; s < substeps; ++s) {
+    bool const island = runs_islands();
+    if (island && warm == SBS_WARM_START_NONE) launch_islands(dt, iterations, substeps, true, false, false);
+    bool const staged = !(island && warm == SBS_WARM_START_NONE);
+    for (uint32_t s = 0; staged && s < substeps; ++s) {
         if (s == 0)
             timed(SBS_KERNEL_PREDICT, V, [&] { launch_predict(stream, xi.p, xn.p, vel.p, V, g0, g1, g2, force, float(dt), block); });
         else
@@ -1050,7 +1197,8 @@ void sbs_gpu::enqueue_frame(double dt_frame, uint32_t iterations, uint32_t subst
                 warmed = true;
             }
         }
-        for (uint32_t it = 0; it < iterations; ++it) {
+        if (island) launch_islands(dt, iterations, 1, false, warmed, fused0 && warmed);
+        for (uint32_t it = 0; !island && it < iterations; ++it) {
             int const first = it == 0;
             if (have_contacts && !(first && fused0 && warmed))
                 timed(SBS_KERNEL_CONTACT, S, [&] {
@@ -1079,7 +1227,7 @@ void sbs_gpu::enqueue_frame(double dt_frame, uint32_t iterations, uint32_t subst
             }
         }
     }
-    timed(SBS_KERNEL_COMMIT, V, [&] { launch_commit(stream, xi.p, xn.p, vel.p, V, float(dt), block); });
+    if (staged) timed(SBS_KERNEL_COMMIT, V, [&] { launch_commit(stream, xi.p, xn.p, vel.p, V, float(dt), block); });
     if (surface_refresh && ntris)  // timestep.cpp:61-66
         launch_surface_refresh(stream, surf.p, xn.p, stris.p, stri_off.p, stri_inc.p, snormal.p, S);
     if (check) enqueue_residual(dt);

@@ -1,5 +1,6 @@
-// Device functions of the time step's kernels: position arithmetic, prediction and velocity update, the
-// Green, stable neo-Hookean and contact projections.
+// Device functions of the time step shared by the kernels that run one stage per launch (kernels.hip)
+// and those that run a whole frame of a small body in one launch (island.hip): position arithmetic,
+// prediction and velocity update, the Green, stable neo-Hookean and contact projections.
 #pragma once
 #include <type_traits>
 
