@@ -162,23 +162,30 @@ __device__ inline double grid_eval(sdf_dev const& f, double px, double py, doubl
     return phi;
 }
 
-// Mesh data of the node-distance kernel: non-degenerate triangles (3 vertex ids) and the
-// pseudonormals of vertices, edges (3 per triangle: (0,1), (1,2), (2,0)) and faces, indexed by
-// triangle; the triangles' corner positions (9 doubles each) in a spatial order with the original
-// index of each, and the bounding boxes (lo xyz, hi xyz) of tiles of consecutive triangles in
-// that order.
+// Mesh data of the node-distance kernels: the non-degenerate triangles, their corners in a spatial order
+// and the tree of bounding boxes over that order, the normals that give the distance its sign.
+constexpr uint32_t kTreeArity = 4, kTreeLevels = 16;  // 4^16 triangles
 struct mesh_dev {
-    const uint32_t* tri;
-    const double* corners;
-    const double* vnormal;
-    const double* enormal;
-    const double* fnormal;
-    const uint32_t* orig;
-    const double* tile_box;
-    uint32_t m, ntiles;
+    const uint32_t* tri;      // 3 vertices per triangle, original order
+    const double* corners;    // 9 per triangle, Morton order
+    const double* vnormal;    // angle-weighted sums per vertex
+    const double* fnormal;    // unit normals, original order
+    const uint32_t* orig;     // Morton order -> original triangle
+    const uint32_t* face_off; // vertex -> its triangles, increasing (original order)
+    const uint32_t* faces;
+    // for the tests of the walk, in FP32 relative to `center`: every tree node, level after level from the
+    // leaves up, as (box lo, n.x), (box hi, n.y), (n.z, lowest and highest corner . n, with n the mean unit
+    // normal of its triangles) and a word that says where its children are; and the triangles' corners
+    const float4* node;
+    const float4* corners32;
+    double center[3];
+    float reach;              // largest coordinate relative to the center
+    uint32_t level_off[kTreeLevels], level_count[kTreeLevels];
+    uint32_t levels;          // tree levels; a leaf holds kTreeArity consecutive triangles, a node as many children
+    uint32_t m;
 };
 
-void launch_grid_nodes(hipStream_t s, mesh_dev mesh, const uint32_t res[3], const double dmin[3],
+void launch_grid_nodes(hipStream_t s, mesh_dev const& mesh, const uint32_t res[3], const double dmin[3],
                        const double cell[3], double* nodes);
 
 // Host side: argument checks, cell size, the node values of a triangle mesh's signed distance
