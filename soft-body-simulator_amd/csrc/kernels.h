@@ -182,6 +182,8 @@ void launch_jp_round(hipStream_t s, uint32_t n, uint32_t arity, const uint32_t* 
 void launch_jp_keys(hipStream_t s, uint32_t n, const uint32_t* prev, uint64_t* key, int block);
 
 void launch_copy_pos(hipStream_t s, const pos4* a, pos4* b, uint32_t n);
+// x, y, z of n positions and n velocities to packed arrays (pinned host memory); a null output is left out.
+void launch_pack_state(hipStream_t s, const pos4* x, const float4* v, uint32_t n, double* xo, float* vo);
 
 // The warm-start network's side of a hex group's warm-start pass: per tet (execution order) the
 // multiplier history hist (the pair one substep before the stored one) and the body-size feature;

@@ -142,6 +142,18 @@ __global__ void k_copy_pos(const pos4* __restrict__ a, pos4* __restrict__ b, uin
     if (i < n) b[i] = a[i];
 }
 
+// One component a thread, so that a wave's stores to host memory are one run of 512 (256) bytes; bounded
+// by the link to the host.
+__global__ void __launch_bounds__(256) k_pack_state(const pos4* __restrict__ x, const float4* __restrict__ v,
+                                                    uint32_t n, double* __restrict__ xo, float* __restrict__ vo)
+{
+    std::size_t const i = std::size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= 3 * std::size_t(n)) return;
+    std::size_t const p = i / 3, c = i % 3;
+    if (xo) xo[i] = reinterpret_cast<const double*>(x)[4 * p + c];
+    if (vo) vo[i] = reinterpret_cast<const float*>(v)[4 * p + c];
+}
+
 // ---------------------------------------------------------------- clustered Gauss-Seidel
 
 // One thread per cluster: the cluster's particles are staged in LDS (slot-major, so that the
@@ -1319,6 +1331,11 @@ void launch_hex_capture(hipStream_t s, tet_group_dev g, const uint4* cinfo, cons
     if (!rows) return;
     k_hex_capture<<<grid_for(rows, 256), 256, 0, s>>>(g, cinfo, rowof, raw, stride, offset, inv_dt2, ds_x, ds_t, base,
                                                       rows);
+}
+
+void launch_pack_state(hipStream_t s, const pos4* x, const float4* v, uint32_t n, double* xo, float* vo)
+{
+    if (n) k_pack_state<<<grid_for(3 * n, 256), 256, 0, s>>>(x, v, n, xo, vo);
 }
 
 void launch_copy_pos(hipStream_t s, const pos4* a, pos4* b, uint32_t n)
