@@ -308,9 +308,9 @@ int sbs_gpu_energy(sbs_gpu* sim, double out[6]);
 #define SBS_KERNEL_WARM_START 7 /* features, network inference and the warm-start pass */
 #define SBS_KERNEL_COUNT 8
 
-/* 1: bracket every launch with HIP events on the simulation's stream (not with graphs). A scene of small
- * bodies then runs one launch per stage, as larger ones do (the same results), so that every kind has
- * launches of its own. */
+/* 1: bracket every launch with HIP events on the simulation's stream (not with graphs). A scene whose
+ * frames run several stages in a launch then runs one launch per stage (the same results), so that every
+ * kind has launches of its own. */
 int sbs_gpu_set_timing(sbs_gpu* sim, int enable);
 /* Per kernel kind since the last reset: launches, summed launch time (ms), summed work units
  * (constraints, contacts or particles). Waits for the device. */

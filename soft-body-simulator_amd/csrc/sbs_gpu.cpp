@@ -22,6 +22,7 @@
 #include "contact_hash.h"
 #include "grid_sdf.h"
 #include "island.h"
+#include "tile.h"
 #include "kernels.h"
 #include "scan_sort.h"
 #include "mlp.h"
@@ -182,6 +183,18 @@ struct sbs_gpu {
     void plan_islands();
     bool runs_islands() const { return islands.n && !timing && !(cap_net && cap_stride); }
     void launch_islands(double dt, uint32_t iterations, uint32_t substeps, bool whole, bool warmed, bool contacts_done);
+
+    // several colors per launch (tile.hip); not ready when a launch per color is the faster way
+    tile_plan tiles;
+    dev_buf<pos4> xi_other;    // the second position array of a sweep
+    dev_buf<float> clam_other;  // and the second contact multipliers
+    void plan_tiles(std::vector<pos4> const& x);
+    bool runs_tiles(uint32_t iterations, int warm) const
+    {
+        // a warm-started sweep reads the group's multipliers in its first iteration and writes them in its last
+        return tiles.ready() && !timing && !(cap_net && cap_stride) && (iterations > 1 || warm == SBS_WARM_START_NONE);
+    }
+    void launch_tiles(double dt, uint32_t iterations, bool warmed, bool contacts_done, contact_dev c);
 
     int block = 256;
     int cluster_block = 64;
@@ -853,6 +866,7 @@ void sbs_gpu::commit(uint32_t recolor_passes)
         if (bodies_collide) setup_body_contacts(tr, x);
     }
     plan_islands();
+    plan_tiles(x);
     hip_check(hipStreamSynchronize(stream), "commit");
     committed = true;
 }
@@ -963,6 +977,180 @@ void sbs_gpu::launch_islands(double dt, uint32_t iterations, uint32_t substeps, 
     island_dev const d{islands.p, island_stages.p, island_list.p, uint32_t(islands.n), g->ncolors,
                        island_largest, g->largest_stage};
     launch_island_frame(stream, d, g->kind, g->hex, g->tet(), g->clusters(), xi.p, xn.p, vel.p, contacts(), p);
+}
+
+// Tile of each particle: body by body, the particles cut into slabs of equal count along one axis, each slab
+// along the next, each of those along the third; about `wanted` tiles in all.
+static uint32_t cut_tiles(std::vector<body_t> const& bodies, std::vector<pos4> const& x, uint32_t wanted,
+                          std::vector<uint32_t>& tile_of)
+{
+    tile_of.assign(x.size(), 0);
+    uint32_t base = 0;
+    std::vector<uint32_t> order(x.size()), next(x.size());
+    auto at = [&](uint32_t v, int d) { return d == 0 ? x[v].x : (d == 1 ? x[v].y : x[v].z); };
+    constexpr int kBins = 1024;
+    // order[b, e) along axis d in g runs of about equal count (particles of one bin stay together); their starts
+    auto cut = [&](uint32_t b, uint32_t e, int d, uint32_t g) {
+        std::vector<uint32_t> starts(g + 1, e);
+        starts[0] = b;
+        if (g == 1 || e - b < 2) return starts;
+        double lo = 1e300, hi = -1e300;
+        for (uint32_t i = b; i < e; ++i) lo = std::min(lo, at(order[i], d)), hi = std::max(hi, at(order[i], d));
+        double const scale = hi > lo ? (kBins - 1) / (hi - lo) : 0.0;
+        auto bin = [&](uint32_t v) { return int(std::min(double(kBins - 1), std::max(0.0, (at(v, d) - lo) * scale + 0.5))); };
+        std::array<uint32_t, kBins + 1> first{};
+        for (uint32_t i = b; i < e; ++i) ++first[bin(order[i]) + 1];
+        for (int k = 0; k < kBins; ++k) first[k + 1] += first[k];
+        std::array<uint32_t, kBins> fill;
+        std::copy(first.begin(), first.end() - 1, fill.begin());
+        for (uint32_t i = b; i < e; ++i) next[b + fill[bin(order[i])]++] = order[i];
+        std::copy(next.begin() + b, next.begin() + e, order.begin() + b);
+        for (uint32_t k = 1, q = 0; k < g; ++k) {
+            uint64_t const want = uint64_t(e - b) * k / g;
+            while (q < kBins && first[q + 1] <= want) ++q;
+            bool const up = q < kBins && first[q + 1] - want < want - first[q];
+            starts[k] = std::max(starts[k - 1], b + first[up ? q + 1 : q]);
+        }
+        return starts;
+    };
+    for (auto const& body : bodies) {
+        if (!body.n) continue;
+        double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300}, len[3], volume = 1.0;
+        for (uint32_t i = 0; i < body.n; ++i)
+            for (int d = 0; d < 3; ++d) {
+                lo[d] = std::min(lo[d], at(body.offset + i, d));
+                hi[d] = std::max(hi[d], at(body.offset + i, d));
+            }
+        int dims = 0;
+        for (int d = 0; d < 3; ++d)
+            if (hi[d] > lo[d]) volume *= hi[d] - lo[d], ++dims;
+        double const spacing = dims ? std::pow(volume / body.n, 1.0 / dims) : 1.0;
+        for (int d = 0; d < 3; ++d) len[d] = (hi[d] - lo[d]) / spacing + 1.0;
+        uint32_t const most = std::max<uint32_t>(1, uint32_t(std::llround(double(wanted) * body.n / double(x.size()))));
+        // the split whose tiles, with a rim of some particles around, are the smallest
+        uint32_t g[3] = {1, 1, 1};
+        double best = 1e300;
+        for (uint32_t a = 1; a <= most; ++a)
+            for (uint32_t b = 1; a * b <= most; ++b) {
+                uint32_t const c = most / (a * b);
+                double const size = (len[0] / a + 3.0) * (len[1] / b + 3.0) * (len[2] / c + 3.0);
+                if (size < best) best = size, g[0] = a, g[1] = b, g[2] = c;
+            }
+        uint32_t const b0 = body.offset, e0 = body.offset + body.n;
+        std::iota(order.begin() + b0, order.begin() + e0, b0);
+        auto const sx = cut(b0, e0, 0, g[0]);
+        for (uint32_t i = 0; i < g[0]; ++i) {
+            auto const sy = cut(sx[i], sx[i + 1], 1, g[1]);
+            for (uint32_t j = 0; j < g[1]; ++j) {
+                auto const sz = cut(sy[j], sy[j + 1], 2, g[2]);
+                for (uint32_t k = 0; k < g[2]; ++k)
+                    if (sz[k] < sz[k + 1]) {
+                        for (uint32_t q = sz[k]; q < sz[k + 1]; ++q) tile_of[order[q]] = base;
+                        ++base;
+                    }
+            }
+        }
+    }
+    return base;
+}
+
+// Plans the tiles if they are the faster way, by the estimated time of an iteration. A tile's stage takes
+// (measured, us) 3.3 + 0.0022 n for n <= 256 hex cells of neo-Hookean tets, 13.6 + 0.006 n of Green tets, 0.85 +
+// 0.0003 n and 2.6 + 0.002 n for single tets; a launch 2.9 + 0.0017 p beside its stages, p particles in the
+// largest tile. A launch per color takes 5.1, 15.3, 3.6 and 5.0 us and 0.16, 0.12, 0.1 and 0.1 us per 1,000
+// elements, the contacts 2 us more. One tile per compute unit: 512 tiles run two to a unit and share its
+// issue slots (1M tets 7.6 ms for four frames against 6.3; 2M 71.6 us an iteration against 74.9). Colors per
+// launch, 8, 4 or 2: with more, fewer launches but wider rims (129k tets 32.8, 34.8 and 40.6 us an iteration,
+// 384k 59, 47 and 53). The plan adds 1-2 ms to a commit of 2-7 ms, 5 ms to one of 67 (1M tets).
+void sbs_gpu::plan_tiles(std::vector<pos4> const& x)
+{
+    group_t const* g = nullptr;
+    for (auto const& o : groups)
+        if (o.count) {
+            if (g) return;
+            g = &o;
+        }
+    if (!g || islands.n || g->kind == 2 || g->count >= kTileConstraints || !(g->hex || !g->clustered())) return;
+    if (uint64_t(g->ncolors) * V >= (uint64_t(1) << 28)) return;
+    int const type = (g->hex ? 0 : 2) + (g->kind == 0 ? 1 : 0);
+    constexpr double stage_us[4] = {3.3, 13.6, 0.85, 2.6}, instance_us[4] = {0.0022, 0.006, 0.0003, 0.002};
+    constexpr double launch_us[4] = {5.1, 15.3, 3.6, 5.0}, element_us[4] = {0.16e-3, 0.12e-3, 0.1e-3, 0.1e-3};
+    std::vector<uint32_t> const& first = g->hex ? g->cluster_color_offsets : g->color_offsets;
+    double best = S && slots ? 2.0 : 0.0;
+    for (uint32_t c = 0; c < g->ncolors; ++c) best += launch_us[type] + element_us[type] * (first[c + 1] - first[c]);
+    try {
+        std::vector<uint32_t> tile_of, bounds;
+        uint32_t const n = cut_tiles(bodies, x, std::min<uint32_t>(256, 1 + V / 64), tile_of);
+        tile_source const src{V, g->num_elements(), g->ncolors, g->hex, g->hex ? g->cl_v0.p : g->idx.p, g->cl_v1.p,
+                              first.data(), g->color_offsets.data(), surface_of_dev.p, tile_of.data(), n};
+        tile_scratch scratch(stream, src);
+        for (uint32_t per : {8u, 4u, 2u}) {
+            uint32_t const nseg = (g->ncolors + per - 1) / per;
+            std::vector<uint32_t> b(nseg + 1);
+            for (uint32_t k = 0; k <= nseg; ++k) b[k] = uint32_t(uint64_t(g->ncolors) * k / nseg);
+            tile_counts const counts = scratch.count(b);
+            double us = 0.0;
+            for (uint32_t k = 0; k < nseg; ++k) {
+                uint32_t largest = 0;
+                for (uint32_t t = 0; t < n; ++t) largest = std::max(largest, counts.particles[std::size_t(k) * n + t]);
+                us += largest <= kTileParticles ? 2.9 + 0.0017 * largest : 1e30;
+            }
+            for (uint32_t c = 0; us < best && c < g->ncolors; ++c) {
+                uint32_t m = 0;
+                for (uint32_t t = 0; t < n; ++t) m = std::max(m, counts.instances[std::size_t(t) * g->ncolors + c]);
+                us += stage_us[type] * ((m + kTileBlock - 1) / kTileBlock) + instance_us[type] * m;
+            }
+            if (us < best)
+                best = us, bounds = b;
+            else if (!bounds.empty())
+                break;
+            if (g->ncolors <= per / 2) break;
+        }
+        if (bounds.empty()) return;
+        scratch.build(bounds, scratch.count(bounds), tiles);
+        xi_other.alloc(V);
+        if (S && slots) clam_other.alloc(std::size_t(S) * slots);
+    } catch (api_error const& e) {
+        if (e.code != SBS_ERR_OUT_OF_MEMORY) throw;
+        (void)hipGetLastError();
+        tiles = tile_plan{};  // a launch per color needs none of it
+        xi_other.release();
+        clam_other.release();
+    }
+}
+
+// The iterations of one substep between its prediction and its velocity update, from xi back to xi.
+void sbs_gpu::launch_tiles(double dt, uint32_t iterations, bool warmed, bool contacts_done, contact_dev c)
+{
+    group_t const* g = nullptr;
+    for (auto const& o : groups)
+        if (o.count) g = &o;
+    double const dt2 = dt * dt, at = g->alpha / dt2;
+    tile_params p{};
+    p.contact_at = float(params.collision_compliance / dt2);
+    p.alpha_tilde = float(at);
+    p.gamma = float(at * (g->beta * dt2) / dt);
+    p.inv_dt2 = float(1.0 / dt2);
+    p.beta_dt = float(g->beta * dt);
+    pos4 *from = xi.p, *to = xi_other.p;
+    bool const have_contacts = S && slots;
+    float* lam[2] = {clam.p, clam_other.p};
+    for (uint32_t it = 0; it < iterations; ++it) {
+        for (std::size_t k = 0; k < tiles.segments.size(); ++k) {
+            p.zero = it == 0 && !warmed;
+            p.from_group = it == 0 && warmed;
+            p.to_group = it + 1 == iterations;
+            p.contacts = k == 0 && have_contacts && !(it == 0 && contacts_done);
+            p.first_contacts = it == 0;
+            // the last iteration's contact multipliers end in the contacts' own array
+            int const out = int((iterations - 1 - it) & 1);
+            p.lambda_out = lam[out];
+            c.lambda = lam[out ^ 1];
+            launch_tile_segment(stream, tiles, k, g->kind, g->hex, g->tet(), from, to, xn.p, c, p);
+            std::swap(from, to);
+        }
+    }
+    if (from != xi.p) launch_copy_pos(stream, from, xi.p, V);
 }
 
 void sbs_gpu::detect()
@@ -1202,6 +1390,7 @@ void sbs_gpu::enqueue_frame(double dt_frame, uint32_t iterations, uint32_t subst
     bool const island = runs_islands();
     if (island && warm == SBS_WARM_START_NONE) launch_islands(dt, iterations, substeps, true, false, false);
     bool const staged = !(island && warm == SBS_WARM_START_NONE);
+    bool const tiled = !island && runs_tiles(iterations, warm);
     for (uint32_t s = 0; staged && s < substeps; ++s) {
         if (s == 0)
             timed(SBS_KERNEL_PREDICT, V, [&] { launch_predict(stream, xi.p, xn.p, vel.p, V, g0, g1, g2, force, float(dt), block); });
@@ -1242,11 +1431,13 @@ void sbs_gpu::enqueue_frame(double dt_frame, uint32_t iterations, uint32_t subst
                     warm_net_dev wn{g.ws_hist.p, g.ws_bsize.p, capture ? g.ws_raw.p : nullptr,
                                     learned ? ws_net->pack.p : nullptr, learned ? ws_net->bias.p : nullptr,
                                     learned ? ws_net->norm.p : nullptr};
+                    contact_dev wc = c;  // the array the sweep's second iteration reads
+                    if (tiled && !(iterations & 1)) wc.lambda = clam_other.p;
                     timed(SBS_KERNEL_WARM_START, g.count, [&] {
                         launch_hex_warm_start(stream, g.tet(), g.clusters(), xtilde, xi.p, g.ws_cinfo.p,
                                               g.ws_rows, float(1.0 / dt2), mode == kApplyExplicit,
                                               make_float2(float(ws_scale), float(ws_scale_hyd)), g.ws_disp.p,
-                                              g.ws_csr_off.p, g.ws_csr.p, V, fused0 ? surface_of_dev.p : nullptr, c,
+                                              g.ws_csr_off.p, g.ws_csr.p, V, fused0 ? surface_of_dev.p : nullptr, wc,
                                               c_at, prow.p, uint32_t(prow.n), net_mode, wn);
                     }, 2);
                 } else {
@@ -1256,7 +1447,8 @@ void sbs_gpu::enqueue_frame(double dt_frame, uint32_t iterations, uint32_t subst
             }
         }
         if (island) launch_islands(dt, iterations, 1, false, warmed, fused0 && warmed);
-        for (uint32_t it = 0; !island && it < iterations; ++it) {
+        if (tiled) launch_tiles(dt, iterations, warmed, fused0 && warmed, c);
+        for (uint32_t it = 0; !island && !tiled && it < iterations; ++it) {
             int const first = it == 0;
             if (have_contacts && !(first && fused0 && warmed))
                 timed(SBS_KERNEL_CONTACT, S, [&] {

@@ -47,6 +47,15 @@ __device__ __forceinline__ void loads_issued()
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// A workgroup barrier that orders LDS only. __syncthreads also waits for every global load and store in
+// flight, the next stage's prefetched data among them.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // a - b of two positions, rounded to FP32
 __device__ __forceinline__ v3 sub(pos4 a, pos4 b)
 {
@@ -376,9 +385,11 @@ __device__ __forceinline__ float contact_slot(pos4& P, pos4 q, v3 n, float w, fl
     return lm + dl;
 }
 
-// Slots [k0, cnt) of vertex s.
+// Slots [k0, cnt) of vertex s. snap(r): the position of surface vertex r that triangle contacts refer to;
+// set(slot, lm) takes the updated multiplier, which is read from c.lambda.
+template <class Snap, class Set>
 __device__ __forceinline__ void contact_slots(contact_dev const& c, pos4& P, uint32_t s, uint32_t k0, uint32_t cnt,
-                                              float alpha_tilde, bool first)
+                                              float alpha_tilde, bool first, Snap&& snap, Set&& set)
 {
     float const w = wof(P);
     for (uint32_t k = k0; k < cnt; ++k) {
@@ -388,14 +399,21 @@ __device__ __forceinline__ void contact_slots(contact_dev const& c, pos4& P, uin
         float wt = 0.0f;
         if (c.snap && q.w >= double(c.nsdf)) {  // a surface triangle: its closest point as it is now
             uint4 const tr = c.btris[uint32_t(q.w) - c.nsdf];
-            pos4 const a = c.snap[tr.x], b = c.snap[tr.y], d = c.snap[tr.z];
+            pos4 const a = snap(tr.x), b = snap(tr.y), d = snap(tr.z);
             wt = float(q.x * q.x * a.w + q.y * q.y * b.w + q.z * q.z * d.w);
             double const hx = c.body_h * double(n.x), hy = c.body_h * double(n.y), hz = c.body_h * double(n.z);
             q = make_double4(q.x * a.x + q.y * b.x + q.z * d.x + hx, q.x * a.y + q.y * b.y + q.z * d.y + hy,
                              q.x * a.z + q.y * b.z + q.z * d.z + hz, q.w);
         }
-        c.lambda[slot] = contact_slot(P, q, n, w, wt, alpha_tilde, first ? 0.0f : c.lambda[slot]);
+        set(slot, contact_slot(P, q, n, w, wt, alpha_tilde, first ? 0.0f : c.lambda[slot]));
     }
+}
+
+__device__ __forceinline__ void contact_slots(contact_dev const& c, pos4& P, uint32_t s, uint32_t k0, uint32_t cnt,
+                                              float alpha_tilde, bool first)
+{
+    contact_slots(c, P, s, k0, cnt, alpha_tilde, first, [&](uint32_t r) { return c.snap[r]; },
+                  [&](uint32_t slot, float lm) { c.lambda[slot] = lm; });
 }
 
 __device__ __forceinline__ void contact_vertex_at(contact_dev const& c, pos4& P, uint32_t s, float alpha_tilde,
