@@ -5,22 +5,29 @@
 namespace sbs {
 
 // LDS of a compute unit a workgroup may use for positions, and the bytes a particle takes there (three
-// FP64 coordinates and its FP32 inverse mass); some hundred bytes are left for the kernels' own.
+// FP64 coordinates and its FP32 inverse mass); the rest holds the chunks, 16 bytes each, and the kernels' own
+// words.
 constexpr std::size_t kIslandLds = 160 * 1024, kIslandBytes = 28;
-constexpr uint32_t kIslandParticles = uint32_t((kIslandLds - 512) / kIslandBytes);
+constexpr uint32_t kIslandChunks = 320;
+constexpr uint32_t kIslandParticles = uint32_t((kIslandLds - 512 - 16 * kIslandChunks) / kIslandBytes);
 // Constraints of a scene of islands: 16-byte offsets into its arrays fit 32 bits.
 constexpr uint32_t kIslandConstraints = 1u << 28;
 
 // The islands of a scene whose single constraint group is laid out island by island inside each color.
 struct island_dev {
-    const uint4* islands;  // first particle, particles, first surface vertex, surface vertices
-    const uint4* stages;   // [island][color]: first element, first constraint, constraint stride of a
-                           // cluster's tets, elements
+    const uint4* islands;  // 2 a piece: first particle, particles, first surface vertex, surface vertices;
+                           // first chunk, chunks, 0, 0
+    const uint4* chunks;   // up to a workgroup's elements of one color: first element, first constraint,
+                           // constraint stride of a cluster's tets, elements (top bit: the color ends here)
     uint32_t* clist;       // scratch, one word per surface vertex
-    uint32_t count, ncolors;
-    uint32_t cap;            // particles of the largest island (the stride of its LDS arrays)
-    uint32_t largest_stage;  // elements of the largest stage of any island
+    uint32_t count;
+    uint32_t cap;         // particles of the largest island (the stride of its LDS arrays)
+    uint32_t chunks_cap;  // chunks of the island with the most
+    uint32_t block;       // elements of a chunk, threads of a workgroup: island_block()
 };
+
+// 256 threads keep a wave to a SIMD; more where a stage of an island (largest: its elements) has more.
+constexpr uint32_t island_block(bool hex, uint32_t largest) { return largest <= 256 ? 256 : (hex ? 512 : 1024); }
 
 struct solve_params {
     uint32_t substeps, iterations;

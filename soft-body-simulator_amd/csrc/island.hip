@@ -4,12 +4,15 @@
 // one launch per stage.
 //
 // What bounds it: the chain of stages. A stage is one color's constraints of the island, at most a
-// few waves, so its time is one wave's dependent arithmetic (about 2.6 us for the six neo-Hookean
+// few waves, so its time is one wave's dependent arithmetic (about 2.8 us for the six neo-Hookean
 // tets of a hex cell, 0.45 us for one tet) plus the exchange with the next stage: through LDS and a
 // barrier here, through a kernel boundary and two memory round trips when every stage is a launch
 // (5.4-6.5 us a stage whatever its size). The next stage's particle ids, material and multipliers
-// are loaded into the registers that the running stage has just used, so they are there when its
-// barrier opens.
+// are loaded into the registers that the running stage has just used, and nothing waits for them before
+// their use: the records of the chunks lie in LDS, the barrier orders LDS only, the sweep has no branch
+// that some waves take. (With records from memory, __syncthreads and a skip for waves without an element,
+// the compiler waited for all loads in flight three times a stage: a frame of the demo bar 361 us now and
+// 405 then, 864 hex cells 902 and 960.)
 //
 // The stages and their order are those of the per-launch path, each element is projected by the same
 // device functions, and elements of one color share no particle: positions, velocities and
@@ -24,6 +27,7 @@ namespace {
 
 using lds_double = __attribute__((address_space(3))) double;
 using lds_float = __attribute__((address_space(3))) float;
+using lds_uint = __attribute__((address_space(3))) uint32_t;
 
 // The island's working positions: one LDS array per coordinate and one of the FP32 inverse masses. 32-byte
 // rows (two 16-byte accesses) had fewer addresses but more bank conflicts: the corners of one color's
@@ -31,6 +35,11 @@ using lds_float = __attribute__((address_space(3))) float;
 struct island_pos {
     lds_double *x, *y, *z;
     lds_float* w;
+    lds_uint* chunk;  // 4 words a chunk
+    __device__ __forceinline__ uint4 record(uint32_t k) const
+    {
+        return uniform(make_uint4(chunk[4 * k], chunk[4 * k + 1], chunk[4 * k + 2], chunk[4 * k + 3]));
+    }
     __device__ __forceinline__ pos4 get(uint32_t l) const { return make_double4(x[l], y[l], z[l], double(w[l])); }
     __device__ __forceinline__ void put(uint32_t l, pos4 p) const
     {
@@ -44,50 +53,33 @@ __device__ __forceinline__ island_pos island_lds(uint32_t cap)
 {
     extern __shared__ double lds[];
     lds_double* const x = (lds_double*)lds;
-    return {x, x + cap, x + 2 * cap, (lds_float*)(lds + 3 * std::size_t(cap))};
+    lds_float* const w = (lds_float*)(x + 3 * cap);
+    return {x, x + cap, x + 2 * cap, w, (lds_uint*)(w + cap)};
 }
 
-// Where the sweep over the island's stages is: color c with its record (first element, first
-// constraint, constraint stride between a cluster's tets, elements of the island) and the chunk of
-// `block` elements in it.
-struct island_cursor {
-    uint32_t c, q;
-    uint4 rec;
-};
-
-// Moves to the next chunk with elements; returns true when it starts the sweep again.
-__device__ __forceinline__ bool advance(island_cursor& k, const uint4* __restrict__ st, uint32_t ncolors, uint32_t block)
-{
-    if ((k.q + 1) * block < k.rec.w) {
-        ++k.q;
-        return false;
-    }
-    bool wrapped = false;
-    k.q = 0;
-    do {
-        if (++k.c == ncolors) k.c = 0, wrapped = true;
-        k.rec = st[k.c];
-    } while (k.rec.w == 0);
-    return wrapped;
-}
+// A chunk's lane: its element, or the last one for lanes past the end.
+__device__ __forceinline__ uint32_t chunk_size(uint4 rec) { return rec.w & 0x7fffffffu; }
+__device__ __forceinline__ uint32_t chunk_lane(uint4 rec) { return min(threadIdx.x, chunk_size(rec) - 1u); }
 
 // The frame (or the part of it that p names) around the sweep: per-particle passes, contacts, and
-// `item(cursor now, cursor next, next one starts from zero multipliers)` for every chunk of every
-// stage, with a barrier after the last chunk of a stage.
-template <int BLOCK, class Start, class Item>
+// `item(chunk now, chunk next, now starts from zero multipliers)` for every chunk of every stage, with a
+// barrier after the last chunk of a stage. ids(chunk), data(chunk): load the first item's.
+template <int BLOCK, class Data, class Item>
 __device__ __forceinline__ void run_island(island_dev const& d, pos4* xi, pos4* xn, float4* v, contact_dev const& c,
-                                           solve_params const& p, island_pos const& P, uint4 isl, Start&& start,
+                                           solve_params const& p, island_pos const& P, uint4 isl, Data&& data,
                                            Item&& item)
 {
     __shared__ uint32_t nlist;  // surface vertices of the island that hold contacts
     uint32_t const tid = threadIdx.x;
-    const uint4* __restrict__ st = d.stages + std::size_t(blockIdx.x) * d.ncolors;
-    island_cursor now{0, 0, make_uint4(0, 0, 0, 0)};
-    while (now.c < d.ncolors && (now.rec = st[now.c]).w == 0) ++now.c;
-    bool const work = now.c < d.ncolors && p.iterations > 0;
-    if (work) start(now, p.zero_first != 0);
+    uint4 const where = uniform(d.islands[2 * blockIdx.x + 1]);
+    const uint32_t* __restrict__ recs = reinterpret_cast<const uint32_t*>(d.chunks + where.x);
+    uint32_t const n = where.y;
+    bool const work = n && p.iterations > 0;
+    for (uint32_t k = tid; k < 4 * n; k += BLOCK) P.chunk[k] = recs[k];
     if (tid == 0) nlist = 0;
     __syncthreads();
+    uint4 now = work ? P.record(0) : uint4{};
+    if (work) data(now);
     if (c.S && c.slots)
         for (uint32_t s = isl.z + tid; s < isl.z + isl.w; s += BLOCK)
             if (c.count[s]) d.clist[isl.z + atomicAdd(&nlist, 1u)] = s;
@@ -143,15 +135,13 @@ __device__ __forceinline__ void run_island(island_dev const& d, pos4* xi, pos4* 
                     contact_vertex_at(c, x, s, p.contact_at, it == 0);
                     P.put(l, x);
                 }
-                __syncthreads();
+                lds_barrier();
             }
-            if (!work) continue;
-            for (bool wrapped = false; !wrapped;) {
-                island_cursor next = now;
-                wrapped = advance(next, st, d.ncolors, BLOCK);
-                bool const zero = p.zero_first && (wrapped ? it + 1 == p.iterations : it == 0);
+            bool const zero = p.zero_first && it == 0;
+            for (uint32_t k = 0; work && k < n; ++k) {
+                uint4 const next = P.record(k + 1 < n ? k + 1 : 0);
                 item(now, next, zero);
-                if (next.q == 0) __syncthreads();  // the stage's last chunk
+                if (now.w >> 31) lds_barrier();
                 now = next;
             }
         }
@@ -179,86 +169,75 @@ template <int KIND, bool DAMPED, int BLOCK>
 __global__ void __launch_bounds__(BLOCK, 2) k_island_hex(island_dev d, tet_group_dev g, cluster_dev cl, pos4* xi, pos4* xn,
                                                       float4* v, contact_dev c, solve_params p)
 {
-    uint4 const isl = d.islands[blockIdx.x];
+    uint4 const isl = uniform(d.islands[2 * blockIdx.x]);
     island_pos const P = island_lds(d.cap);
     float4 A[kHexTets], B[kHexTets];
     float4 G[KIND == 0 ? kHexTets : 1];
     float2 C[KIND == 0 ? 1 : kHexTets], L[kHexTets];
     int4 va, vb;
-    auto element = [&](island_cursor const& k, bool& active) {
-        uint32_t const e = k.q * BLOCK + threadIdx.x;
-        active = e < k.rec.w;
-        return active ? e : k.rec.w - 1;
-    };
     // t: the constraint's index, its 16-byte offset in a 32-bit register (a scene of islands has fewer
     // than 2^28 constraints): one vector addition a tet, where a scalar 64-bit base per tet and array took
     // 230 scalar instructions a stage, each an issue slot of a wave that has its SIMD to itself
-    auto load = [&](uint32_t t, int m, bool zero) {
+    auto load = [&](uint32_t t, int m) {
         A[m] = lane_load(g.m0, t);
         B[m] = lane_load(g.m1, t);
         if (KIND == 0) {
             G[m] = lane_load(g.m2, t);
-            float const l = lane_load(g.lambda, t);
-            L[m].x = zero ? 0.0f : l;
+            L[m].x = lane_load(g.lambda, t);
         } else {
             C[m] = lane_load(reinterpret_cast<const float2*>(g.m2), t);
-            float2 const l = lane_load(reinterpret_cast<const float2*>(g.lambda), t);
-            L[m] = zero ? make_float2(0.0f, 0.0f) : l;
+            L[m] = lane_load(reinterpret_cast<const float2*>(g.lambda), t);
         }
     };
-    auto load_ids = [&](island_cursor const& k, uint32_t e) {
-        va = lane_load(cl.v0, k.rec.x + e);
-        vb = lane_load(cl.v1, k.rec.x + e);
+    auto load_ids = [&](uint4 rec) {
+        va = lane_load(cl.v0, rec.x + chunk_lane(rec));
+        vb = lane_load(cl.v1, rec.x + chunk_lane(rec));
     };
-    auto start = [&](island_cursor const& k, bool zero) {
-        bool active;
-        uint32_t const e = element(k, active);
-        load_ids(k, e);
+    auto data = [&](uint4 rec) {
+        load_ids(rec);
 #pragma unroll
-        for (int m = 0; m < kHexTets; ++m) load(k.rec.y + uint32_t(m) * k.rec.z + e, m, zero);
+        for (int m = 0; m < kHexTets; ++m) load(rec.y + uint32_t(m) * rec.z + chunk_lane(rec), m);
     };
-    auto item = [&](island_cursor const& now, island_cursor const& next, bool zero) {
-        bool active, later;
-        uint32_t const e = element(now, active), en = element(next, later);
-        if (!__any(active)) {
-            load_ids(next, en);
-#pragma unroll
-            for (int m = 0; m < kHexTets; ++m) load(next.rec.y + uint32_t(m) * next.rec.z + en, m, zero);
-            return;
-        }
+    auto item = [&](uint4 now, uint4 next, bool zero) {
+        bool const active = threadIdx.x < chunk_size(now);
         uint32_t const l[8] = {va.x - isl.x, va.y - isl.x, va.z - isl.x, va.w - isl.x,
                                vb.x - isl.x, vb.y - isl.x, vb.z - isl.x, vb.w - isl.x};
-        load_ids(next, en);
         pos4 X[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) X[k] = P.get(l[k]);
+        loads_issued();
+        load_ids(next);
+        loads_issued();
+        uint32_t const t0 = now.y + chunk_lane(now), n0 = next.y + chunk_lane(next);
 #pragma unroll
         for (int m = 0; m < kHexTets; ++m) {
             int const s0 = kHexSlots[m][0], s1 = kHexSlots[m][1], s2 = kHexSlots[m][2], s3 = kHexSlots[m][3];
             pos4 Q[4] = {X[s0], X[s1], X[s2], X[s3]};
             uint32_t const id[4] = {l[s0], l[s1], l[s2], l[s3]};
             auto xn_of = [&](int k) { return xn[isl.x + id[k]]; };
-            uint32_t const t = now.rec.y + uint32_t(m) * now.rec.z + e;
+            uint32_t const t = t0 + uint32_t(m) * now.z;
+            float2 lm = zero ? make_float2(0.0f, 0.0f) : L[m];
             if (KIND == 0) {
-                green_project(Q, xn_of, A[m], B[m], G[m], p.alpha_tilde, DAMPED ? p.gamma : 0.0f, L[m].x);
-                if (active) lane_store(g.lambda, t, L[m].x);
+                green_project(Q, xn_of, A[m], B[m], G[m], p.alpha_tilde, DAMPED ? p.gamma : 0.0f, lm.x);
+                if (active) lane_store(g.lambda, t, lm.x);
             } else {
-                neohookean_project<DAMPED>(Q, xn_of, A[m], B[m], C[m], p.inv_dt2, p.beta_dt, L[m]);
-                if (active) lane_store(reinterpret_cast<float2*>(g.lambda), t, L[m]);
+                neohookean_project<DAMPED>(Q, xn_of, A[m], B[m], C[m], p.inv_dt2, p.beta_dt, lm);
+                if (active) lane_store(reinterpret_cast<float2*>(g.lambda), t, lm);
             }
             X[s0] = Q[0];
             X[s1] = Q[1];
             X[s2] = Q[2];
             X[s3] = Q[3];
-            load(next.rec.y + uint32_t(m) * next.rec.z + en, m, zero);
+            if (m == kHexTets - 1 && active) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) P.put(l[k], X[k]);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // the registers are free: no use of them sinks past the loads
+            load(n0 + uint32_t(m) * next.z, m);
             loads_issued();
         }
-        if (active) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) P.put(l[k], X[k]);
-        }
     };
-    run_island<BLOCK>(d, xi, xn, v, c, p, P, isl, start, item);
+    run_island<BLOCK>(d, xi, xn, v, c, p, P, isl, data, item);
 }
 
 // One constraint per lane (tets without clusters).
@@ -266,49 +245,48 @@ template <int KIND, bool DAMPED, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) k_island_tets(island_dev d, tet_group_dev g, pos4* xi, pos4* xn, float4* v,
                                                        contact_dev c, solve_params p)
 {
-    uint4 const isl = d.islands[blockIdx.x];
+    uint4 const isl = uniform(d.islands[2 * blockIdx.x]);
     island_pos const P = island_lds(d.cap);
     int4 id;
     float4 A, B, G;
     float2 C, L;
-    auto load = [&](island_cursor const& k, bool zero) {
-        uint32_t const e = k.q * BLOCK + threadIdx.x, t = k.rec.y + (e < k.rec.w ? e : k.rec.w - 1);
+    auto data = [&](uint4 rec) {
+        uint32_t const t = rec.y + chunk_lane(rec);
         id = lane_load(g.idx, t);
         A = lane_load(g.m0, t);
         B = lane_load(g.m1, t);
         if (KIND == 0) {
             G = lane_load(g.m2, t);
-            float const l = lane_load(g.lambda, t);
-            L.x = zero ? 0.0f : l;
+            L.x = lane_load(g.lambda, t);
         } else {
             C = lane_load(reinterpret_cast<const float2*>(g.m2), t);
-            float2 const l = lane_load(reinterpret_cast<const float2*>(g.lambda), t);
-            L = zero ? make_float2(0.0f, 0.0f) : l;
+            L = lane_load(reinterpret_cast<const float2*>(g.lambda), t);
         }
     };
-    auto item = [&](island_cursor const& now, island_cursor const& next, bool zero) {
-        uint32_t const e = now.q * BLOCK + threadIdx.x;
-        if (e < now.rec.w) {
-            uint32_t const t = now.rec.y + e;
-            uint32_t const l[4] = {id.x - isl.x, id.y - isl.x, id.z - isl.x, id.w - isl.x};
-            pos4 Q[4] = {P.get(l[0]), P.get(l[1]), P.get(l[2]), P.get(l[3])};
-            auto xn_of = [&](int k) { return xn[isl.x + l[k]]; };
-            bool moved = true;
-            if (KIND == 0) {
-                moved = green_project(Q, xn_of, A, B, G, p.alpha_tilde, DAMPED ? p.gamma : 0.0f, L.x);
-                lane_store(g.lambda, t, L.x);
-            } else {
-                neohookean_project<DAMPED>(Q, xn_of, A, B, C, p.inv_dt2, p.beta_dt, L);
-                lane_store(reinterpret_cast<float2*>(g.lambda), t, L);
-            }
-            if (moved) {
+    auto item = [&](uint4 now, uint4 next, bool zero) {
+        bool const active = threadIdx.x < chunk_size(now);
+        uint32_t const t = now.y + chunk_lane(now);
+        uint32_t const l[4] = {id.x - isl.x, id.y - isl.x, id.z - isl.x, id.w - isl.x};
+        pos4 Q[4] = {P.get(l[0]), P.get(l[1]), P.get(l[2]), P.get(l[3])};
+        auto xn_of = [&](int k) { return xn[isl.x + l[k]]; };
+        bool moved = true;
+        float2 lm = zero ? make_float2(0.0f, 0.0f) : L;
+        if (KIND == 0) {
+            moved = green_project(Q, xn_of, A, B, G, p.alpha_tilde, DAMPED ? p.gamma : 0.0f, lm.x);
+            if (active) lane_store(g.lambda, t, lm.x);
+        } else {
+            neohookean_project<DAMPED>(Q, xn_of, A, B, C, p.inv_dt2, p.beta_dt, lm);
+            if (active) lane_store(reinterpret_cast<float2*>(g.lambda), t, lm);
+        }
+        if (active && moved) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) P.put(l[k], Q[k]);
-            }
+            for (int k = 0; k < 4; ++k) P.put(l[k], Q[k]);
         }
-        load(next, zero);
+        __builtin_amdgcn_sched_barrier(0);
+        data(next);
+        loads_issued();
     };
-    run_island<BLOCK>(d, xi, xn, v, c, p, P, isl, load, item);
+    run_island<BLOCK>(d, xi, xn, v, c, p, P, isl, data, item);
 }
 
 template <class K, class... Args>
@@ -328,8 +306,8 @@ void launch_island_frame(hipStream_t s, island_dev const& d, int kind, bool hex,
                          solve_params const& p)
 {
     if (!d.count) return;
-    std::size_t const lds = std::size_t(d.cap) * kIslandBytes;
-    bool const wide = d.largest_stage > 256, damped = kind == 0 ? p.gamma != 0.0f : p.beta_dt != 0.0f;
+    std::size_t const lds = std::size_t(d.cap) * kIslandBytes + std::size_t(d.chunks_cap) * 16;
+    bool const wide = d.block > 256, damped = kind == 0 ? p.gamma != 0.0f : p.beta_dt != 0.0f;
     auto hexes = [&](auto kernel, int block) { launch_island(s, kernel, d.count, block, lds, d, g, cl, xi, xn, v, c, p); };
     auto tets = [&](auto kernel, int block) { launch_island(s, kernel, d.count, block, lds, d, g, xi, xn, v, c, p); };
     if (hex) {

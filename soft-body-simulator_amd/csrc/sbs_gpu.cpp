@@ -177,9 +177,9 @@ struct sbs_gpu {
     void setup_body_contacts(std::vector<uint4> const& tr, std::vector<pos4> const& x);
 
     // whole-frame launches (island.hip): one workgroup per body; no rows when the scene has none
-    dev_buf<uint4> islands, island_stages;
+    dev_buf<uint4> islands, island_chunks;
     dev_buf<uint32_t> island_list;
-    uint32_t island_largest = 0;
+    uint32_t island_largest = 0, island_most_chunks = 0;
     void plan_islands();
     bool runs_islands() const { return islands.n && !timing && !(cap_net && cap_stride); }
     void launch_islands(double dt, uint32_t iterations, uint32_t substeps, bool whole, bool warmed, bool contacts_done);
@@ -496,8 +496,11 @@ void sbs_gpu::color_group(group_t& g, uint32_t recolor_passes)
 // at 256), 5.4-5.8 up to 512, 7.6 up to 640, and the bodies share 256 compute units. Measured: 24x6x6 cells
 // 6.2 us a stage launched, 3.7 here; one body of 512 cells a color 5.1 launched, 5.8 here; 512 bodies of 2,900
 // to 6,500 tets 12.3 and 5.6; 512 bodies of 8,000 to 14,000 tets 26.9 and 9.9. Green cells: 13.5-16 us
-// launched; 11.6-12.5 here up to 256 cells, 16.5 at 512. Single tets: 2.1-4.9 us launched, 1.05-1.9
-// (neo-Hookean) and 2.4-4.6 (Green) here at any size that fits LDS.
+// launched; 11.6-12.5 here up to 256 cells, 16.5 at 512. Single tets are compared with the launches that run
+// several colors in tiles, 1.3 us a stage (neo-Hookean) and 2.65 (Green) at 24,600 tets, 3.1 and 8 at 1M; here,
+// with n elements a stage, 0.70 + 0.0014 n, and 1.85 + 0.0018 n (Green; with more than 256 in a stage, at 1,024
+// threads, 4.2 + 0.0009 n). One body of 4,374, 10,368 and 24,576 tets, us an iteration here and in tiles:
+// neo-Hookean 30.5 and 45.7, 40.1 and 47.7, 59.1 and 49.5; Green 75 and 94, 160 and 96, 172 and 99.
 bool sbs_gpu::small_bodies(group_t const& g) const
 {
     if (g.kind == 2 || body_contacts || g.count >= kIslandConstraints) return false;
@@ -514,8 +517,19 @@ bool sbs_gpu::small_bodies(group_t const& g) const
             if (g.body_of(c) != b) return false;  // a cluster over two bodies
         ++counts[std::size_t(b) * g.ncolors + g.color[c0]];
     }
-    if (!g.clustered()) return true;
     double longest = 0.0, sum = 0.0;
+    if (!g.clustered()) {
+        uint32_t const most = *std::max_element(counts.begin(), counts.end());
+        for (std::size_t b = 0; b < bodies.size(); ++b) {
+            uint32_t n = 0;
+            for (uint32_t c = 0; c < g.ncolors; ++c) n += counts[b * g.ncolors + c];
+            double const mean = double(n) / g.ncolors;
+            double const us = g.kind == 1 ? 0.70 + 0.0014 * mean : most <= 256 ? 1.85 + 0.0018 * mean : 4.2 + 0.0009 * mean;
+            longest = std::max(longest, us);
+            sum += us;
+        }
+        return std::max(longest, sum / 256.0) < (g.kind == 1 ? 1.3 + 1.9e-6 * ne : 2.65 + 5.8e-6 * ne);
+    }
     for (std::size_t b = 0; b < bodies.size(); ++b) {
         uint32_t n = 0;
         for (uint32_t c = 0; c < g.ncolors; ++c) n = std::max(n, counts[b * g.ncolors + c]);
@@ -926,27 +940,38 @@ void sbs_gpu::plan_islands()
     for (auto const& o : groups)
         if (o.count) g = &o;
     if (!g || g->body_stages.empty()) return;
-    std::vector<uint4> rec;
+    std::vector<uint4> rec, chunks;
     std::vector<uint64_t> work(bodies.size(), 0);
-    uint32_t base = 0;
+    uint32_t base = 0, largest = 0, most = 0;
+    uint32_t const block = island_block(g->hex, g->largest_stage);
     for (std::size_t b = 0; b < bodies.size(); ++b) {
         rec.push_back(make_uint4(bodies[b].offset, bodies[b].n, base, uint32_t(bodies[b].surface.size())));
         base += uint32_t(bodies[b].surface.size());
-        island_largest = std::max(island_largest, bodies[b].n);
+        largest = std::max(largest, bodies[b].n);
         for (uint32_t c = 0; c < g->ncolors; ++c) work[b] += g->body_stages[b * g->ncolors + c].w;
     }
     // the longest first: workgroups start in order, and the last ones to end should be short
     std::vector<uint32_t> order(bodies.size());
     std::iota(order.begin(), order.end(), 0u);
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return work[a] > work[b]; });
-    std::vector<uint4> sorted, stages;
+    std::vector<uint4> sorted;
     for (uint32_t b : order) {
+        uint32_t const first = uint32_t(chunks.size());
+        for (uint32_t c = 0; c < g->ncolors; ++c) {
+            uint4 const st = g->body_stages[std::size_t(b) * g->ncolors + c];
+            for (uint32_t q = 0; q < st.w; q += block)
+                chunks.push_back(make_uint4(st.x + q, st.y + q, st.z,
+                                            std::min(block, st.w - q) | (q + block >= st.w ? 0x80000000u : 0u)));
+        }
+        most = std::max(most, uint32_t(chunks.size()) - first);
         sorted.push_back(rec[b]);
-        stages.insert(stages.end(), g->body_stages.begin() + std::size_t(b) * g->ncolors,
-                      g->body_stages.begin() + (std::size_t(b) + 1) * g->ncolors);
+        sorted.push_back(make_uint4(first, uint32_t(chunks.size()) - first, 0, 0));
     }
+    if (most > kIslandChunks) return;  // a mesh of many tets a particle: its chunks leave no room beside it
+    island_largest = largest;
+    island_most_chunks = most;
     islands.upload(sorted.data(), sorted.size(), stream);
-    island_stages.upload(stages.data(), stages.size(), stream);
+    island_chunks.upload(chunks.data(), chunks.size(), stream);
     island_list.alloc(std::max<uint32_t>(S, 1));
     hip_check(hipStreamSynchronize(stream), "upload islands");
 }
@@ -974,8 +999,8 @@ void sbs_gpu::launch_islands(double dt, uint32_t iterations, uint32_t substeps, 
     p.gamma = float(at * (g->beta * dt2) / dt);
     p.inv_dt2 = float(1.0 / dt2);
     p.beta_dt = float(g->beta * dt);
-    island_dev const d{islands.p, island_stages.p, island_list.p, uint32_t(islands.n), g->ncolors,
-                       island_largest, g->largest_stage};
+    island_dev const d{islands.p,      island_chunks.p,    island_list.p, uint32_t(islands.n / 2),
+                       island_largest, island_most_chunks, island_block(g->hex, g->largest_stage)};
     launch_island_frame(stream, d, g->kind, g->hex, g->tet(), g->clusters(), xi.p, xn.p, vel.p, contacts(), p);
 }
 
@@ -1071,7 +1096,7 @@ void sbs_gpu::plan_tiles(std::vector<pos4> const& x)
             g = &o;
         }
     if (!g || islands.n || g->kind == 2 || g->count >= kTileConstraints || !(g->hex || !g->clustered())) return;
-    if (uint64_t(g->ncolors) * V >= (uint64_t(1) << 28)) return;
+    if (uint64_t(g->ncolors) * V >= (uint64_t(1) << 28) || V > 256 * kTileParticles) return;
     int const type = (g->hex ? 0 : 2) + (g->kind == 0 ? 1 : 0);
     constexpr double stage_us[4] = {3.3, 13.6, 0.85, 2.6}, instance_us[4] = {0.0022, 0.006, 0.0003, 0.002};
     constexpr double launch_us[4] = {5.1, 15.3, 3.6, 5.0}, element_us[4] = {0.16e-3, 0.12e-3, 0.1e-3, 0.1e-3};
@@ -1080,7 +1105,10 @@ void sbs_gpu::plan_tiles(std::vector<pos4> const& x)
     for (uint32_t c = 0; c < g->ncolors; ++c) best += launch_us[type] + element_us[type] * (first[c + 1] - first[c]);
     try {
         std::vector<uint32_t> tile_of, bounds;
-        uint32_t const n = cut_tiles(bodies, x, std::min<uint32_t>(256, 1 + V / 64), tile_of);
+        uint32_t const wanted = std::min<uint32_t>(256, 1 + V / 64);
+        uint32_t n = cut_tiles(bodies, x, wanted, tile_of);
+        if (n > 256) n = cut_tiles(bodies, x, uint32_t(uint64_t(wanted) * wanted / n), tile_of);
+        double const rounds = double((n + 255) / 256);
         tile_source const src{V, g->num_elements(), g->ncolors, g->hex, g->hex ? g->cl_v0.p : g->idx.p, g->cl_v1.p,
                               first.data(), g->color_offsets.data(), surface_of_dev.p, tile_of.data(), n};
         tile_scratch scratch(stream, src);
@@ -1100,6 +1128,7 @@ void sbs_gpu::plan_tiles(std::vector<pos4> const& x)
                 for (uint32_t t = 0; t < n; ++t) m = std::max(m, counts.instances[std::size_t(t) * g->ncolors + c]);
                 us += stage_us[type] * ((m + kTileBlock - 1) / kTileBlock) + instance_us[type] * m;
             }
+            us *= rounds;
             if (us < best)
                 best = us, bounds = b;
             else if (!bounds.empty())

@@ -47,6 +47,13 @@ __device__ __forceinline__ void loads_issued()
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// A record that every lane holds, in scalar registers.
+__device__ __forceinline__ uint4 uniform(uint4 r)
+{
+    auto word = [](uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); };
+    return make_uint4(word(r.x), word(r.y), word(r.z), word(r.w));
+}
+
 // A workgroup barrier that orders LDS only. __syncthreads also waits for every global load and store in
 // flight, the next stage's prefetched data among them.
 __device__ __forceinline__ void lds_barrier()

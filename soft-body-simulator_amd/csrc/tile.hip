@@ -39,13 +39,6 @@ struct tile_dev {
     uint32_t tiles, per, cap, instances;
 };
 
-// A record that every lane holds, in scalar registers.
-__device__ __forceinline__ uint4 uniform(uint4 r)
-{
-    auto word = [](uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); };
-    return make_uint4(word(r.x), word(r.y), word(r.z), word(r.w));
-}
-
 struct tile_lds {
     lds_double *x, *y, *z, *w;
     lds_float* f;     // the inverse masses again, in FP32

@@ -33,6 +33,21 @@ def _loose_point(sc):
     return sc
 
 
+def _many(n, tets_of, kind):
+    """n bodies of one mesh, a constraint per tet, side by side."""
+    x0, tets = tets_of
+    sc = scenes.Scene("islands", gravity_is_force=False, coloring="hash")
+    s2t, tris = S.boundary(len(x0), tets)
+    step = np.array([float(np.ptp(x0[:, 0])) + 1.0, 0.0, 0.0])
+    for k in range(n):
+        sc.bodies.append(scenes.Body(x0=x0 + k * step, tets=tets, mass=S.lumped_mass(x0, tets, 1000.0), surface=s2t,
+                                     triangles=tris))
+    sc.groups.append(scenes.Group(kind, np.repeat(np.arange(n, dtype=np.uint32), len(tets)), np.tile(tets, (n, 1)),
+                                  alpha=1e-4, young=np.full(n * len(tets), 2e5), poisson=np.full(n * len(tets), 0.3)))
+    sc.planes.append(((0.0, 1.0, 0.0), (0.0, 0.01, 0.0), (-1e30,) * 3, (1e30,) * 3))
+    return sc
+
+
 CASES = {
     # elements of a stage: under one wave, one to four waves, colors that some bodies have no element of;
     # hex_wide's and batch_wide's stages have more than 256 (workgroups of 512 threads)
@@ -48,6 +63,8 @@ CASES = {
     # more elements in a stage than 256 lanes
     "tets_wide": lambda: _single(S.box6(13, 13, 11, 0.1), "neohookean", False, spheres=4),
     "tets_green_wide": lambda: _single(S.box6(12, 12, 10, 0.1), "green", False, spheres=4),
+    # the same where there are enough bodies that one workgroup each is the faster way
+    "tets_green_wide_many": lambda: _many(45, S.box6(12, 12, 10, 0.1), "green"),
     # bodies from one cell up, boxes and ellipsoids
     "batch": lambda: scenes.batch(9, (6.0, 9000.0), seed=4, young_range=(1e4, 1e5), drop_range=(-0.01, 0.0)),
     # up to 5,800 particles and 600 cells of a color in a body, enough bodies that it is worth it
