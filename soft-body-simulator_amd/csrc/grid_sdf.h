@@ -163,16 +163,12 @@ __device__ inline double grid_eval(sdf_dev const& f, double px, double py, doubl
 }
 
 // Mesh data of the node-distance kernels: the non-degenerate triangles, their corners in a spatial order
-// and the tree of bounding boxes over that order, the normals that give the distance its sign.
+// and the tree of bounding boxes over that order.
 constexpr uint32_t kTreeArity = 4, kTreeLevels = 16;  // 4^16 triangles
 struct mesh_dev {
     const uint32_t* tri;      // 3 vertices per triangle, original order
     const double* corners;    // 9 per triangle, Morton order
-    const double* vnormal;    // angle-weighted sums per vertex
-    const double* fnormal;    // unit normals, original order
     const uint32_t* orig;     // Morton order -> original triangle
-    const uint32_t* face_off; // vertex -> its triangles, increasing (original order)
-    const uint32_t* faces;
     // for the tests of the walk, in FP32 relative to `center`: every tree node, level after level from the
     // leaves up, as (box lo, n.x), (box hi, n.y), (n.z, lowest and highest corner . n, with n the mean unit
     // normal of its triangles) and a word that says where its children are; and the triangles' corners
@@ -185,8 +181,13 @@ struct mesh_dev {
     uint32_t m;
 };
 
-void launch_grid_nodes(hipStream_t s, mesh_dev const& mesh, const uint32_t res[3], const double dmin[3],
-                       const double cell[3], double* nodes);
+// The normals that give the distance its sign.
+struct mesh_normals {
+    const double* vnormal;    // angle-weighted sums per vertex
+    const double* fnormal;    // unit normals, original order
+    const uint32_t* face_off; // vertex -> its triangles, increasing (original order)
+    const uint32_t* faces;
+};
 
 // Host side: argument checks, cell size, the node values of a triangle mesh's signed distance
 // written to device memory, environment_body_t's extended domain, and evaluation of one SDF at

@@ -14,14 +14,12 @@
 // the batches. On the 20,480-triangle ball and 24^3 cells (104,625 nodes) 963 us, where the scan of
 // 128-triangle tiles through LDS that it replaces took 12.4 ms.
 #include <algorithm>
-#include <array>
 #include <cmath>
-#include <cstring>
-#include <utility>
 #include <vector>
 
 #include "abi_util.h"
 #include "grid_sdf.h"
+#include "scan_sort.h"
 #include "sdf.h"
 
 namespace sbs {
@@ -116,32 +114,36 @@ __device__ __forceinline__ void wave_nearest(nearest& best)
     }
 }
 
-// The signed distance from the nearest triangle: its closest point again, the pseudo-normal of the
-// feature that holds it (an edge's is the sum of its triangles' unit normals in original order).
-__device__ __forceinline__ double signed_distance(mesh_dev const& mesh, const double p[3], nearest const& best)
+// The signed distance from the nearest triangle t (in Morton order): its closest point again, the
+// pseudo-normal of the feature that holds it (an edge's is the sum of its triangles' unit normals in original
+// order).
+__device__ __forceinline__ double signed_distance(mesh_dev const& mesh, mesh_normals const& nm, const double p[3],
+                                                  uint32_t t)
 {
 #pragma clang fp contract(off)
-    if (best.t == 0xffffffffu) return DBL_MAX;
+    if (t == 0xffffffffu) return DBL_MAX;
     double c[9], q[3], nrm[3] = {0.0, 0.0, 0.0};
-    for (int k = 0; k < 9; ++k) c[k] = mesh.corners[9 * std::size_t(best.t) + k];
+    for (int k = 0; k < 9; ++k) c[k] = mesh.corners[9 * std::size_t(t) + k];
+    uint32_t const o = mesh.orig[t];
     int feat;
     tri_closest_point(p, c, q, &feat);
-    const uint32_t* tv = mesh.tri + 3 * std::size_t(best.o);
+    const uint32_t* tv = mesh.tri + 3 * std::size_t(o);
     if (feat < 3) {
-        for (int d = 0; d < 3; ++d) nrm[d] = mesh.vnormal[3 * std::size_t(tv[feat]) + d];
+        for (int d = 0; d < 3; ++d) nrm[d] = nm.vnormal[3 * std::size_t(tv[feat]) + d];
     } else if (feat < 6) {
         uint32_t const v = tv[feat - 3], w = tv[feat == 5 ? 0 : feat - 2];
-        for (uint32_t i = mesh.face_off[v], e = mesh.face_off[v + 1]; i < e; ++i) {
-            uint32_t const f = mesh.faces[i];
+        for (uint32_t i = nm.face_off[v], e = nm.face_off[v + 1]; i < e; ++i) {
+            uint32_t const f = nm.faces[i];
             const uint32_t* fv = mesh.tri + 3 * std::size_t(f);
             if (fv[0] != w && fv[1] != w && fv[2] != w) continue;
-            for (int d = 0; d < 3; ++d) nrm[d] = nrm[d] + mesh.fnormal[3 * std::size_t(f) + d];
+            for (int d = 0; d < 3; ++d) nrm[d] = nrm[d] + nm.fnormal[3 * std::size_t(f) + d];
         }
     } else {
-        for (int d = 0; d < 3; ++d) nrm[d] = mesh.fnormal[3 * std::size_t(best.o) + d];
+        for (int d = 0; d < 3; ++d) nrm[d] = nm.fnormal[3 * std::size_t(o) + d];
     }
-    double const s = (p[0] - q[0]) * nrm[0] + (p[1] - q[1]) * nrm[1] + (p[2] - q[2]) * nrm[2];
-    double const d = sqrt(best.d2);
+    double const e0 = p[0] - q[0], e1 = p[1] - q[1], e2 = p[2] - q[2];
+    double const s = e0 * nrm[0] + e1 * nrm[1] + e2 * nrm[2];
+    double const d = sqrt(e0 * e0 + e1 * e1 + e2 * e2);
     return s < 0.0 ? -d : d;
 }
 
@@ -151,9 +153,9 @@ __device__ __forceinline__ double signed_distance(mesh_dev const& mesh, const do
 // list whose exact FP64 closest points the lanes then share. (A lane per grid node walked 64 different
 // paths: 4.3 ms on the 20,480-triangle ball and 24^3 cells, 0.96 ms so.) The first bound is exact distances
 // to 64 triangles that are neighbours in Morton order: those of the last node's nearest one, for a run's
-// first node those of the nearest box.
+// first node those of the nearest box. out: the nearest triangle (in Morton order; ~0: none).
 __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_params gp, uint64_t n,
-                                                       double* __restrict__ out)
+                                                       uint32_t* __restrict__ out)
 {
     constexpr uint32_t kWaves = kBlock / 64;
     __shared__ uint32_t stack_lds[kWaves][kStack], list_lds[kWaves][kList];
@@ -162,7 +164,7 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
     if (l0 >= n) return;
     uint32_t const cnt = uint32_t(n - l0 < kRun ? n - l0 : kRun);
     if (mesh.m == 0) {
-        if (lane < cnt) out[l0 + lane] = DBL_MAX;
+        if (lane < cnt) out[l0 + lane] = 0xffffffffu;
         return;
     }
     uint32_t* const stack = stack_lds[wave];
@@ -170,7 +172,7 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
     uint64_t const below = (uint64_t(1) << lane) - 1;
     grid_dims const dims(gp.res);
     uint32_t const top = mesh.levels - 1, start = top < 2 ? top : 2;
-    nearest mine;  // lane r: the nearest of node l0 + r
+    uint32_t mine = 0xffffffffu;  // lane r: the nearest of node l0 + r
     uint32_t block = 0;  // of 64 triangles
     for (uint32_t r = 0; r < cnt; ++r) {
         double p[3];
@@ -235,49 +237,167 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
         drain();
         wave_nearest(best);
         block = best.t < mesh.m ? best.t / 64 : 0;
-        if (lane == r) mine = best;
+        if (lane == r) mine = best.t;
     }
-    if (lane < cnt) {
-        double p[3];
-        grid_node_position(dims, gp.dmin, gp.cell, l0 + lane, p);
-        out[l0 + lane] = signed_distance(mesh, p, mine);
+    if (lane < cnt) out[l0 + lane] = mine;
+}
+
+__global__ void __launch_bounds__(kBlock) k_grid_signs(mesh_dev mesh, mesh_normals nm, grid_params gp, uint64_t n,
+                                                       const uint32_t* __restrict__ nearest_of, double* __restrict__ out)
+{
+    uint64_t const l = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (l >= n) return;
+    double p[3];
+    grid_node_position(grid_dims(gp.res), gp.dmin, gp.cell, l, p);
+    out[l] = signed_distance(mesh, nm, p, nearest_of[l]);
+}
+
+// ---------------------------------------------------------------- the tree
+
+// Morton codes of the triangles' centroids, 10 bits per axis over the mesh's box (lo, scale = 1024 / extent).
+struct morton_box {
+    double lo[3], scale[3];
+};
+
+__global__ void k_tree_keys(const double* __restrict__ pos, const uint32_t* __restrict__ tri, uint32_t m, morton_box box,
+                            uint32_t* __restrict__ key, uint32_t* __restrict__ orig)
+{
+    uint32_t const t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= m) return;
+    uint32_t code = 0;
+    for (int d = 0; d < 3; ++d) {
+        double const c = (pos[3 * std::size_t(tri[3 * t]) + d] + pos[3 * std::size_t(tri[3 * t + 1]) + d] +
+                          pos[3 * std::size_t(tri[3 * t + 2]) + d]) / 3.0;
+        uint32_t x = uint32_t(fmin(1023.0, fmax(0.0, (c - box.lo[d]) * box.scale[d])));
+        x = (x | (x << 16)) & 0x30000ffu;
+        x = (x | (x << 8)) & 0x300f00fu;
+        x = (x | (x << 4)) & 0x30c30c3u;
+        x = (x | (x << 2)) & 0x9249249u;
+        code |= x << d;
+    }
+    key[t] = code;
+    orig[t] = t;
+}
+
+// The triangles' corners in Morton order, and relative to the mesh's center in FP32 (the walk's margin covers
+// the rounding).
+__global__ void k_tree_corners(mesh_dev mesh, const double* __restrict__ pos, double* __restrict__ corners,
+                               float4* __restrict__ corners32)
+{
+    uint32_t const i = blockIdx.x * blockDim.x + threadIdx.x;  // of 3 m
+    if (i >= 3 * mesh.m) return;
+    uint32_t const v = mesh.tri[3 * std::size_t(mesh.orig[i / 3]) + i % 3];
+    double const x = pos[3 * std::size_t(v)], y = pos[3 * std::size_t(v) + 1], z = pos[3 * std::size_t(v) + 2];
+    corners[3 * std::size_t(i)] = x;
+    corners[3 * std::size_t(i) + 1] = y;
+    corners[3 * std::size_t(i) + 2] = z;
+    corners32[i] = make_float4(float(x - mesh.center[0]), float(y - mesh.center[1]), float(z - mesh.center[2]), 0.0f);
+}
+
+__device__ __forceinline__ float wave_min(float v)
+{
+    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// A wave makes a node of tree level `level`: the box of its children (triangles at level 0), and the slab that
+// holds its corners along the mean normal of its triangles, for patches of up to 256 triangles (larger ones
+// bend too far for one). sum: the nodes' summed unit normals.
+__global__ void __launch_bounds__(kBlock) k_tree_level(mesh_dev mesh, uint32_t level, float4* __restrict__ node,
+                                                       float4* __restrict__ sum)
+{
+    uint32_t const i = (blockIdx.x * kBlock + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    if (i >= mesh.level_count[level]) return;
+    uint32_t const n = level ? mesh.level_count[level - 1] : mesh.m, below = level ? mesh.level_off[level - 1] : 0u;
+    uint32_t const j0 = i * kTreeArity, have = min(kTreeArity, n - j0), j = j0 + min(lane, have - 1);
+    float4 l, h, u;
+    if (level == 0) {
+        float4 const a = mesh.corners32[3 * std::size_t(j)], b = mesh.corners32[3 * std::size_t(j) + 1],
+                     c = mesh.corners32[3 * std::size_t(j) + 2];
+        l = make_float4(fminf(a.x, fminf(b.x, c.x)), fminf(a.y, fminf(b.y, c.y)), fminf(a.z, fminf(b.z, c.z)), 0.0f);
+        h = make_float4(fmaxf(a.x, fmaxf(b.x, c.x)), fmaxf(a.y, fmaxf(b.y, c.y)), fmaxf(a.z, fmaxf(b.z, c.z)), 0.0f);
+        float const ex = b.x - a.x, ey = b.y - a.y, ez = b.z - a.z, fx = c.x - a.x, fy = c.y - a.y, fz = c.z - a.z;
+        u = make_float4(ey * fz - ez * fy, ez * fx - ex * fz, ex * fy - ey * fx, 0.0f);
+        float const ln = sqrtf(u.x * u.x + u.y * u.y + u.z * u.z);
+        float const inv = ln > 0.0f && isfinite(ln) ? 1.0f / ln : 0.0f;
+        u = make_float4(inv > 0.0f && isfinite(inv) ? u.x * inv : 0.0f, inv > 0.0f && isfinite(inv) ? u.y * inv : 0.0f,
+                        inv > 0.0f && isfinite(inv) ? u.z * inv : 0.0f, 0.0f);
+    } else {
+        const float4* o = node + 3 * (std::size_t(below) + j);
+        l = o[0];
+        h = o[1];
+        u = sum[below + j];
+    }
+    // of the children, held by the first lanes
+    bool const mine = lane < have;
+    float const lx = wave_min(l.x), ly = wave_min(l.y), lz = wave_min(l.z);
+    float const hx = -wave_min(-h.x), hy = -wave_min(-h.y), hz = -wave_min(-h.z);
+    u = mine ? u : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int o = 2; o > 0; o >>= 1) {
+        u.x += __shfl_xor(u.x, o, 64);
+        u.y += __shfl_xor(u.y, o, 64);
+        u.z += __shfl_xor(u.z, o, 64);
+    }
+    u = make_float4(__shfl(u.x, 0, 64), __shfl(u.y, 0, 64), __shfl(u.z, 0, 64), 0.0f);
+    float const ln = sqrtf(u.x * u.x + u.y * u.y + u.z * u.z);
+    bool const slab = ln > 1e-3f && isfinite(ln) && level < 4;
+    float const gx = slab ? u.x / ln : 0.0f, gy = slab ? u.y / ln : 0.0f, gz = slab ? u.z / ln : 0.0f;
+    float s0 = INFINITY, s1 = INFINITY;  // lowest, and the highest negated
+    if (slab) {
+        std::size_t const per = 3 * std::size_t(kTreeArity) << (2 * level), end = 3 * std::size_t(mesh.m);
+        for (std::size_t k = i * per + lane; k < (i + 1) * per && k < end; k += 64) {
+            float4 const c = mesh.corners32[k];
+            float const e = c.x * gx + c.y * gy + c.z * gz;
+            s0 = fminf(s0, e);
+            s1 = fminf(s1, -e);
+        }
+        s0 = wave_min(s0);
+        s1 = wave_min(s1);
+    }
+    if (lane == 0) {
+        // where its children are: bit 31 a leaf, bits 29-30 their count less one, the rest the leaf's
+        // index or the first child's place in the node array
+        uint32_t const info = (level == 0 ? 0x80000000u | i : below + j0) | (have - 1) << 29;
+        float4* const o = node + 3 * (std::size_t(mesh.level_off[level]) + i);
+        o[0] = make_float4(lx, ly, lz, gx);
+        o[1] = make_float4(hx, hy, hz, gy);
+        o[2] = make_float4(gz, slab ? s0 : -INFINITY, slab ? -s1 : INFINITY, __uint_as_float(info));
+        sum[mesh.level_off[level] + i] = u;
     }
 }
 
 }  // namespace
 
-void launch_grid_nodes(hipStream_t s, mesh_dev const& mesh, const uint32_t res[3], const double dmin[3],
-                       const double cell[3], double* nodes)
-{
-    grid_params gp{};
-    for (int d = 0; d < 3; ++d) {
-        gp.res[d] = res[d];
-        gp.dmin[d] = dmin[d];
-        gp.cell[d] = cell[d];
-    }
-    uint64_t const n = grid_dims(res).nodes(), per_block = uint64_t(kRun) * (kBlock / 64);
-    k_grid_nodes<<<unsigned((n + per_block - 1) / per_block), kBlock, 0, s>>>(mesh, gp, n, nodes);
-}
-
-// Host side of the mesh: non-degenerate triangles, corners and pseudonormals (FP64, no FMA
-// contraction), uploaded to the device.
+// A triangle mesh on the device: its non-degenerate triangles and the tree over them, made there; then the
+// normals that give the distance its sign, made on the host (FP64, no FMA contraction) while the device walks
+// the tree. (The tree made on the host, and everything before the walk: 3.57 ms for the 20,480-triangle ball and
+// 24^3 cells, 1.53 ms so, 0.93 of it the walk.)
 struct mesh_upload {
-    dev_buf<uint32_t> tri, orig, face_off, faces;
-    dev_buf<double> corners, vnormal, fnormal;
-    dev_buf<float4> node, corners32;
+    dev_buf<uint32_t> tri, orig, face_off, faces, key, ws;
+    dev_buf<double> position, corners, vnormal, fnormal;
+    dev_buf<float4> node, corners32, sum;
     mesh_dev view{};
+    std::vector<uint32_t> t;  // vertices of the non-degenerate triangles
+
+    static void cross(const double a[3], const double b[3], double o[3])
+    {
+#pragma clang fp contract(off)
+        o[0] = a[1] * b[2] - a[2] * b[1];
+        o[1] = a[2] * b[0] - a[0] * b[2];
+        o[2] = a[0] * b[1] - a[1] * b[0];
+    }
+    static double dot(const double a[3], const double b[3])
+    {
+#pragma clang fp contract(off)
+        return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
+    }
 
     mesh_upload(hipStream_t s, const double* pos, uint32_t nv, const uint32_t* tris, uint32_t nt)
     {
 #pragma clang fp contract(off)
         auto at = [&](uint32_t v, int d) { return pos[3 * std::size_t(v) + d]; };
-        auto cross = [](const double a[3], const double b[3], double o[3]) {
-            o[0] = a[1] * b[2] - a[2] * b[1];
-            o[1] = a[2] * b[0] - a[0] * b[2];
-            o[2] = a[0] * b[1] - a[1] * b[0];
-        };
-        auto dot = [](const double a[3], const double b[3]) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
-        std::vector<uint32_t> t;
+        double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+        t.reserve(3 * std::size_t(nt));
         for (uint32_t f = 0; f < nt; ++f) {
             double e1[3], e2[3], n[3];
             for (int d = 0; d < 3; ++d) {
@@ -286,17 +406,67 @@ struct mesh_upload {
             }
             cross(e1, e2, n);
             if (dot(n, n) > 0.0)
-                for (int k = 0; k < 3; ++k) t.push_back(tris[3 * f + k]);
+                for (int k = 0; k < 3; ++k) {
+                    t.push_back(tris[3 * f + k]);
+                    for (int d = 0; d < 3; ++d) {
+                        lo[d] = std::min(lo[d], at(tris[3 * f + k], d));
+                        hi[d] = std::max(hi[d], at(tris[3 * f + k], d));
+                    }
+                }
         }
         uint32_t const m = uint32_t(t.size() / 3);
-        std::vector<double> c(9 * std::size_t(m)), vn(3 * std::size_t(nv), 0.0), fn(3 * std::size_t(m));
+        require(m < (1u << 30), "too many triangles");
+        view.m = m;
+        tri.upload(t.data(), t.size(), s);
+        view.tri = tri.p;
+        if (!m) return;
+        morton_box box;
+        for (int d = 0; d < 3; ++d) {
+            box.lo[d] = lo[d];
+            box.scale[d] = hi[d] > lo[d] ? 1024.0 / (hi[d] - lo[d]) : 0.0;
+            view.center[d] = 0.5 * (lo[d] + hi[d]);
+            view.reach = std::max(view.reach, float(0.5 * (hi[d] - lo[d])) * (1.0f + 1e-6f));
+        }
+        uint32_t nodes = 0;
+        for (uint32_t n = m; view.levels < kTreeLevels;) {
+            n = (n + kTreeArity - 1) / kTreeArity;
+            view.level_off[view.levels] = nodes;
+            view.level_count[view.levels++] = n;
+            nodes += n;
+            if (n <= kTreeArity) break;
+        }
+        position.upload(pos, 3 * std::size_t(nv), s);
+        key.alloc(m);
+        orig.alloc(m);
+        ws.alloc(sort_workspace(m));
+        corners.alloc(9 * std::size_t(m));
+        corners32.alloc(3 * std::size_t(m));
+        node.alloc(3 * std::size_t(nodes));
+        sum.alloc(nodes);
+        view.orig = orig.p, view.corners = corners.p, view.corners32 = corners32.p, view.node = node.p;
+        k_tree_keys<<<(m + 255) / 256, 256, 0, s>>>(position.p, tri.p, m, box, key.p, orig.p);
+        radix_sort_pairs(s, key.p, orig.p, m, 30, ws.p);
+        k_tree_corners<<<(3 * m + 255) / 256, 256, 0, s>>>(view, position.p, corners.p, corners32.p);
+        for (uint32_t l = 0; l < view.levels; ++l)
+            k_tree_level<<<(view.level_count[l] + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, s>>>(view, l, node.p, sum.p);
+        hip_check(hipGetLastError(), "mesh tree");
+    }
+
+    // The normals' host arrays stay until the stream has taken them.
+    std::vector<double> vn, fn;
+    std::vector<uint32_t> off, inc;
+
+    mesh_normals normals(hipStream_t s, const double* pos, uint32_t nv)
+    {
+#pragma clang fp contract(off)
+        auto at = [&](uint32_t v, int d) { return pos[3 * std::size_t(v) + d]; };
+        uint32_t const m = view.m;
+        vn.assign(3 * std::size_t(nv), 0.0);
+        fn.resize(3 * std::size_t(m));
         for (uint32_t f = 0; f < m; ++f) {
             double p[3][3];
             for (int k = 0; k < 3; ++k)
-                for (int d = 0; d < 3; ++d) {
-                    p[k][d] = at(t[3 * f + k], d);
-                    c[9 * std::size_t(f) + 3 * k + d] = p[k][d];
-                }
+                for (int d = 0; d < 3; ++d) p[k][d] = at(t[3 * f + k], d);
             double e1[3], e2[3], n[3];
             for (int d = 0; d < 3; ++d) {
                 e1[d] = p[1][d] - p[0][d];
@@ -321,136 +491,17 @@ struct mesh_upload {
             }
         }
         // each vertex's triangles in increasing order
-        std::vector<uint32_t> off(std::size_t(nv) + 1, 0), inc(t.size());
+        off.assign(std::size_t(nv) + 1, 0);
+        inc.resize(t.size());
         for (uint32_t v : t) ++off[v + 1];
         for (std::size_t v = 0; v < nv; ++v) off[v + 1] += off[v];
-        {
-            std::vector<uint32_t> fill(off.begin(), off.end() - 1);
-            for (std::size_t i = 0; i < t.size(); ++i) inc[fill[t[i]]++] = uint32_t(i / 3);
-        }
-        // triangles in Morton order of their centroids (10 bits per axis over the mesh's box),
-        // corners in that order, each with its original index; boxes of every kTreeArity of them, of
-        // every kTreeArity of those, and so on up to at most kTreeArity
-        std::vector<uint32_t> ord(m);
-        {
-            double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-            for (std::size_t i = 0; i < 9 * std::size_t(m); ++i) {
-                lo[i % 3] = std::min(lo[i % 3], c[i]);
-                hi[i % 3] = std::max(hi[i % 3], c[i]);
-            }
-            auto spread = [](uint32_t v) {
-                uint64_t x = v & 0x3ffu;
-                x = (x | (x << 16)) & 0x30000ffull;
-                x = (x | (x << 8)) & 0x300f00full;
-                x = (x | (x << 4)) & 0x30c30c3ull;
-                x = (x | (x << 2)) & 0x9249249ull;
-                return x;
-            };
-            std::vector<std::pair<uint64_t, uint32_t>> key(m);
-            for (uint32_t f = 0; f < m; ++f) {
-                uint64_t code = 0;
-                for (int d = 0; d < 3; ++d) {
-                    double const cen = (c[9 * std::size_t(f) + d] + c[9 * std::size_t(f) + 3 + d] +
-                                        c[9 * std::size_t(f) + 6 + d]) / 3.0;
-                    double const ext = hi[d] - lo[d];
-                    double const u = ext > 0.0 ? (cen - lo[d]) / ext : 0.0;
-                    uint32_t const q = uint32_t(std::min(1023.0, std::max(0.0, u * 1024.0)));
-                    code |= spread(q) << d;
-                }
-                key[f] = {code, f};
-            }
-            std::sort(key.begin(), key.end());
-            for (uint32_t i = 0; i < m; ++i) ord[i] = key[i].second;
-        }
-        std::vector<double> cs(9 * std::size_t(m));
-        for (uint32_t i = 0; i < m; ++i)
-            std::copy(c.begin() + 9 * std::size_t(ord[i]), c.begin() + 9 * std::size_t(ord[i]) + 9,
-                      cs.begin() + 9 * std::size_t(i));
-        // relative to the middle of the mesh's box, in FP32 (the walk's margin covers the rounding)
-        double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-        for (std::size_t i = 0; i < cs.size(); ++i) {
-            lo[i % 3] = std::min(lo[i % 3], cs[i]);
-            hi[i % 3] = std::max(hi[i % 3], cs[i]);
-        }
-        for (int d = 0; d < 3 && m; ++d) {
-            view.center[d] = 0.5 * (lo[d] + hi[d]);
-            view.reach = std::max(view.reach, float(0.5 * (hi[d] - lo[d])) * (1.0f + 1e-6f));
-        }
-        std::vector<float4> c32(3 * std::size_t(m));
-        for (std::size_t i = 0; i < c32.size(); ++i)
-            c32[i] = make_float4(float(cs[3 * i] - view.center[0]), float(cs[3 * i + 1] - view.center[1]),
-                                 float(cs[3 * i + 2] - view.center[2]), 0.0f);
-        std::vector<float4> nd;
-        std::vector<std::array<float, 3>> below(m), sums;  // normals of the triangles, then of the level below
-        for (uint32_t i = 0; i < m; ++i)
-            for (int d = 0; d < 3; ++d) below[i][d] = float(fn[3 * std::size_t(ord[i]) + d]);
-        std::size_t per = 1;  // triangles under a node of the level
-        for (uint32_t n = m, child = 0; n > 0 && view.levels < kTreeLevels; ++view.levels) {
-            uint32_t const cnt = uint32_t((uint64_t(n) + kTreeArity - 1) / kTreeArity), first = uint32_t(nd.size() / 3);
-            nd.resize(nd.size() + 3 * std::size_t(cnt));
-            sums.assign(cnt, {0.0f, 0.0f, 0.0f});
-            per *= kTreeArity;
-            for (uint32_t i = 0; i < cnt; ++i) {
-                float4 l = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
-                float4 h = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-                auto cover = [&](float4 const& a, float4 const& b) {
-                    l = make_float4(std::min(l.x, a.x), std::min(l.y, a.y), std::min(l.z, a.z), 0.0f);
-                    h = make_float4(std::max(h.x, b.x), std::max(h.y, b.y), std::max(h.z, b.z), 0.0f);
-                };
-                std::size_t const j0 = std::size_t(i) * kTreeArity, j1 = std::min<std::size_t>(n, j0 + kTreeArity);
-                std::array<float, 3>& u = sums[i];
-                for (std::size_t j = j0; j < j1; ++j) {
-                    if (view.levels == 0)
-                        for (int k = 0; k < 3; ++k) cover(c32[3 * j + k], c32[3 * j + k]);
-                    else
-                        cover(nd[3 * (child + j)], nd[3 * (child + j) + 1]);
-                    for (int d = 0; d < 3; ++d) u[d] += below[j][d];
-                }
-                float const ln = std::sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-                // slabs for patches of up to 256 triangles; larger ones bend too far for one
-                bool const slab = ln > 1e-3f && std::isfinite(ln) && view.levels < 4;
-                float const g[3] = {slab ? u[0] / ln : 0.0f, slab ? u[1] / ln : 0.0f, slab ? u[2] / ln : 0.0f};
-                float s0 = slab ? INFINITY : -INFINITY, s1 = slab ? -INFINITY : INFINITY;
-                for (std::size_t j = 3 * i * per; slab && j < std::min<std::size_t>(c32.size(), 3 * (i + 1) * per); ++j) {
-                    float const e = c32[j].x * g[0] + c32[j].y * g[1] + c32[j].z * g[2];
-                    s0 = std::min(s0, e);
-                    s1 = std::max(s1, e);
-                }
-                l.w = g[0];
-                h.w = g[1];
-                float4* o = nd.data() + 3 * (std::size_t(first) + i);
-                o[0] = l;
-                o[1] = h;
-                // where its children are: bit 31 a leaf, bits 29-30 their count less one, the rest the leaf's
-                // index or the first child's place in the node array
-                uint32_t const info = (view.levels == 0 ? 0x80000000u | i : child + uint32_t(j0)) |
-                                      (uint32_t(j1 - j0 - 1) << 29);
-                float word;
-                std::memcpy(&word, &info, sizeof word);
-                o[2] = make_float4(g[2], s0, s1, word);
-            }
-            view.level_off[view.levels] = child = first;
-            view.level_count[view.levels] = n = cnt;
-            below.swap(sums);
-            if (cnt <= kTreeArity) {
-                ++view.levels;
-                break;
-            }
-        }
-        tri.upload(t.data(), t.size(), s);
-        corners.upload(cs.data(), cs.size(), s);
-        orig.upload(ord.data(), ord.size(), s);
-        face_off.upload(off.data(), off.size(), s);
-        faces.upload(inc.data(), inc.size(), s);
-        node.upload(nd.data(), nd.size(), s);
-        corners32.upload(c32.data(), c32.size(), s);
+        std::vector<uint32_t> fill(off.begin(), off.end() - 1);
+        for (std::size_t i = 0; i < t.size(); ++i) inc[fill[t[i]]++] = uint32_t(i / 3);
         vnormal.upload(vn.data(), vn.size(), s);
         fnormal.upload(fn.data(), fn.size(), s);
-        hip_check(hipStreamSynchronize(s), "mesh upload");
-        view.tri = tri.p, view.corners = corners.p, view.vnormal = vnormal.p, view.fnormal = fnormal.p;
-        view.orig = orig.p, view.face_off = face_off.p, view.faces = faces.p;
-        view.node = node.p, view.corners32 = corners32.p;
-        view.m = m;
+        face_off.upload(off.data(), off.size(), s);
+        faces.upload(inc.data(), inc.size(), s);
+        return {vnormal.p, fnormal.p, face_off.p, faces.p};
     }
 };
 
@@ -480,11 +531,21 @@ void build_mesh_grid(hipStream_t s, const double* pos, uint32_t nv, const uint32
     require((pos || nv == 0) && (tris || nt == 0), "null mesh argument");
     for (std::size_t i = 0; i < 3 * std::size_t(nt); ++i) require(tris[i] < nv, "triangle vertex index out of range");
     check_grid(dmin, dmax, res);
-    mesh_upload const mesh(s, pos, nv, tris, nt);
-    double cell[3], inv_cell[3];
-    grid_cell_size(dmin, dmax, res, cell, inv_cell);
-    require(mesh.view.m < (1u << 30), "too many triangles");
-    launch_grid_nodes(s, mesh.view, res, dmin, cell, dev_nodes);
+    grid_params gp{};
+    double inv_cell[3];
+    grid_cell_size(dmin, dmax, res, gp.cell, inv_cell);
+    for (int d = 0; d < 3; ++d) {
+        gp.res[d] = res[d];
+        gp.dmin[d] = dmin[d];
+    }
+    uint64_t const n = grid_dims(res).nodes(), per_block = uint64_t(kRun) * (kBlock / 64);
+    dev_buf<uint32_t> nearest_of;
+    nearest_of.alloc(n);
+    mesh_upload mesh(s, pos, nv, tris, nt);
+    k_grid_nodes<<<unsigned((n + per_block - 1) / per_block), kBlock, 0, s>>>(mesh.view, gp, n, nearest_of.p);
+    hip_check(hipGetLastError(), "grid node kernel");
+    mesh_normals const nm = mesh.normals(s, pos, nv);
+    k_grid_signs<<<unsigned((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(mesh.view, nm, gp, n, nearest_of.p, dev_nodes);
     hip_check(hipGetLastError(), "grid node kernel");
     hip_check(hipStreamSynchronize(s), "grid node kernel");
 }
