@@ -1081,8 +1081,8 @@ static uint32_t cut_tiles(std::vector<body_t> const& bodies, std::vector<pos4> c
 
 // Plans the tiles if they are the faster way, by the estimated time of an iteration. A tile's stage takes
 // (measured, us) 3.3 + 0.0022 n for n <= 256 hex cells of neo-Hookean tets, 13.6 + 0.006 n of Green tets, 0.85 +
-// 0.0003 n and 2.6 + 0.002 n for single tets; a launch 2.9 + 0.0017 p beside its stages, p particles in the
-// largest tile. A launch per color takes 5.1, 15.3, 3.6 and 5.0 us and 0.16, 0.12, 0.1 and 0.1 us per 1,000
+// 0.0003 n and 2.6 + 0.002 n for single tets; a tile's launch 2.9 + 0.0017 p beside its stages, with p
+// particles. A launch per color takes 5.1, 15.3, 3.6 and 5.0 us and 0.16, 0.12, 0.1 and 0.1 us per 1,000
 // elements, the contacts 2 us more. One tile per compute unit: 512 tiles run two to a unit and share its
 // issue slots (1M tets 7.6 ms for four frames against 6.3; 2M 71.6 us an iteration against 74.9). Colors per
 // launch, 8, 4 or 2: with more, fewer launches but wider rims (129k tets 32.8, 34.8 and 40.6 us an iteration,
@@ -1119,14 +1119,17 @@ void sbs_gpu::plan_tiles(std::vector<pos4> const& x)
             tile_counts const counts = scratch.count(b);
             double us = 0.0;
             for (uint32_t k = 0; k < nseg; ++k) {
-                uint32_t largest = 0;
-                for (uint32_t t = 0; t < n; ++t) largest = std::max(largest, counts.particles[std::size_t(k) * n + t]);
-                us += largest <= kTileParticles ? 2.9 + 0.0017 * largest : 1e30;
-            }
-            for (uint32_t c = 0; us < best && c < g->ncolors; ++c) {
-                uint32_t m = 0;
-                for (uint32_t t = 0; t < n; ++t) m = std::max(m, counts.instances[std::size_t(t) * g->ncolors + c]);
-                us += stage_us[type] * ((m + kTileBlock - 1) / kTileBlock) + instance_us[type] * m;
+                double longest = 0.0;
+                for (uint32_t t = 0; t < n; ++t) {
+                    uint32_t const p = counts.particles[std::size_t(k) * n + t];
+                    double tile = p <= kTileParticles ? 2.9 + 0.0017 * p : 1e30;
+                    for (uint32_t c = b[k]; c < b[k + 1]; ++c) {
+                        uint32_t const m = counts.instances[std::size_t(t) * g->ncolors + c];
+                        tile += stage_us[type] * ((m + kTileBlock - 1) / kTileBlock) + instance_us[type] * m;
+                    }
+                    longest = std::max(longest, tile);
+                }
+                us += longest;
             }
             us *= rounds;
             if (us < best)

@@ -99,14 +99,14 @@ __device__ __forceinline__ void run_tile(tile_dev const& d, const pos4* __restri
         uint32_t const l0 = base + tid;
 #pragma unroll
         for (uint32_t k = 0; k < kBatch; ++k)
-            if (base + k * kTileBlock < blk.y) e[k] = lane_load(d.particles + blk.x, min(l0 + k * kTileBlock, blk.y - 1));
+            if (base + k * kTileThreads < blk.y) e[k] = lane_load(d.particles + blk.x, min(l0 + k * kTileThreads, blk.y - 1));
     };
     // (without contacts, or for an inner particle, some word: a load under a condition would be waited for)
     const uint32_t* const counts = p.contacts ? c.count : d.elems;
     auto load_rows = [&](uint32_t base) {
 #pragma unroll
         for (uint32_t k = 0; k < kBatch; ++k) {
-            if (base + k * kTileBlock >= blk.y) continue;
+            if (base + k * kTileThreads >= blk.y) continue;
             x[k] = in[e[k].x & ~kTopBit];
             cnt[k] = counts[p.contacts && e[k].y != kNone ? e[k].y : 0u];
         }
@@ -116,10 +116,10 @@ __device__ __forceinline__ void run_tile(tile_dev const& d, const pos4* __restri
         uint32_t const l0 = base + tid;
 #pragma unroll
         for (uint32_t k = 0; k < kBatch; ++k) {
-            if (base + k * kTileBlock >= blk.y) continue;
-            bool const real = l0 + k * kTileBlock < blk.y;
-            uint32_t const l = slot_of(l0 + k * kTileBlock);
-            if (real && p.contacts && e[k].y != kNone && cnt[k]) touched |= 1u << (l0 / kTileBlock + k);
+            if (base + k * kTileThreads >= blk.y) continue;
+            bool const real = l0 + k * kTileThreads < blk.y;
+            uint32_t const l = slot_of(l0 + k * kTileThreads);
+            if (real && p.contacts && e[k].y != kNone && cnt[k]) touched |= 1u << (l0 / kTileThreads + k);
             if (real) {
                 P.put(l, x[k]);
                 P.w[l] = x[k].w;
@@ -128,24 +128,25 @@ __device__ __forceinline__ void run_tile(tile_dev const& d, const pos4* __restri
             }
         }
     };
+    bool const runs = __builtin_amdgcn_readfirstlane(int(tid)) < kTileBlock;
     load_entries(0);
-    ids(first, second);
+    if (runs) ids(first, second);
     uint32_t const rec = recs[min(tid, 4 * n - 1)];
     loads_issued();
     load_rows(0);
-    data(first);
+    if (runs) data(first);
     loads_issued();
     if (tid < 4 * n) P.chunk[tid] = rec;
-    for (uint32_t k = tid + kTileBlock; k < 4 * n; k += kTileBlock) P.chunk[k] = recs[k];
+    for (uint32_t k = tid + kTileThreads; k < 4 * n; k += kTileThreads) P.chunk[k] = recs[k];
     put_rows(0);
-    for (uint32_t base = kBatch * kTileBlock; base < blk.y; base += kBatch * kTileBlock) {
+    for (uint32_t base = kBatch * kTileThreads; base < blk.y; base += kBatch * kTileThreads) {
         load_entries(base);
         load_rows(base);
         put_rows(base);
     }
-    static_assert(kTileParticles <= 32 * kTileBlock, "a bit per particle of a thread");
+    static_assert(kTileParticles <= 32 * kTileThreads, "a bit per particle of a thread");
     for (; touched; touched &= touched - 1) {
-        uint32_t const k = tid + (uint32_t(__ffs(int(touched))) - 1u) * kTileBlock, l = slot_of(k);
+        uint32_t const k = tid + (uint32_t(__ffs(int(touched))) - 1u) * kTileThreads, l = slot_of(k);
         uint2 const q = d.particles[blk.x + k];
         pos4 y = make_double4(P.x[l], P.y[l], P.z[l], P.w[l]);
         contact_slots(c, y, q.y, 0, c.count[q.y], p.contact_at, p.first_contacts != 0,
@@ -154,21 +155,26 @@ __device__ __forceinline__ void run_tile(tile_dev const& d, const pos4* __restri
         P.put(l, y);
     }
     __syncthreads();
-    uint4 now = P.record(0), next = P.record(min(1u, n - 1));
-    for (uint32_t k = 0; k < n; ++k) {
-        uint4 const after = P.record(min(k + 2, n - 1));
-        item(now, next, after);
-        if (now.w) lds_barrier();
-        now = next;
-        next = after;
+    if (runs) {
+        uint4 now = P.record(0), next = P.record(min(1u, n - 1));
+        for (uint32_t k = 0; k < n; ++k) {
+            uint4 const after = P.record(min(k + 2, n - 1));
+            item(now, next, after);
+            if (now.w) lds_barrier();
+            now = next;
+            next = after;
+        }
+    } else {  // the waves that only carry particles
+        for (uint32_t k = 0; k < n; ++k)
+            if (P.record(k).w) lds_barrier();
     }
-    for (uint32_t l0 = tid; l0 < blk.y; l0 += 4 * kTileBlock) {
+    for (uint32_t l0 = tid; l0 < blk.y; l0 += 4 * kTileThreads) {
         uint32_t id[4];
         pos4 o[4];
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            uint32_t const l = slot_of(min(l0 + k * kTileBlock, blk.y - 1));
-            id[k] = l0 + k * kTileBlock < blk.y ? P.id[l] : 0u;
+            uint32_t const l = slot_of(min(l0 + k * kTileThreads, blk.y - 1));
+            id[k] = l0 + k * kTileThreads < blk.y ? P.id[l] : 0u;
             o[k] = make_double4(P.x[l], P.y[l], P.z[l], P.w[l]);
         }
 #pragma unroll
@@ -180,7 +186,7 @@ __device__ __forceinline__ void run_tile(tile_dev const& d, const pos4* __restri
 // Hex-cell clusters, a lane each. No branch in the sweep but the masks of its stores: where one skipped the
 // arithmetic of waves without a cluster, the compiler waited for every load in flight at its join.
 template <int KIND, bool DAMPED>
-__global__ void __launch_bounds__(kTileBlock, 2) k_tile_hex(tile_dev d, tet_group_dev g, const pos4* __restrict__ in,
+__global__ void __launch_bounds__(kTileThreads, 2) k_tile_hex(tile_dev d, tet_group_dev g, const pos4* __restrict__ in,
                                                             pos4* __restrict__ out, const pos4* __restrict__ xn,
                                                             contact_dev c, tile_params p)
 {
@@ -260,7 +266,7 @@ __global__ void __launch_bounds__(kTileBlock, 2) k_tile_hex(tile_dev d, tet_grou
 
 // One constraint per lane (tets without clusters).
 template <int KIND, bool DAMPED>
-__global__ void __launch_bounds__(kTileBlock) k_tile_tets(tile_dev d, tet_group_dev g, const pos4* __restrict__ in,
+__global__ void __launch_bounds__(kTileThreads, 2) k_tile_tets(tile_dev d, tet_group_dev g, const pos4* __restrict__ in,
                                                           pos4* __restrict__ out, const pos4* __restrict__ xn,
                                                           contact_dev c, tile_params p)
 {
@@ -622,7 +628,7 @@ void launch_tile_segment(hipStream_t s, tile_plan const& plan, std::size_t segme
     std::size_t const lds = std::size_t(seg.cap) * kTileBytes + std::size_t(seg.chunks) * 16;
     auto run = [&](auto kernel) {
         allow_lds(reinterpret_cast<const void*>(kernel), lds);
-        kernel<<<per * kXcds, kTileBlock, lds, s>>>(d, g, in, out, xn, c, p);
+        kernel<<<per * kXcds, kTileThreads, lds, s>>>(d, g, in, out, xn, c, p);
     };
     bool const damped = kind == 0 ? p.gamma != 0.0f : p.beta_dt != 0.0f;
     if (hex && kind == 0)
