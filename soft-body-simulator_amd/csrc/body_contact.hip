@@ -317,8 +317,13 @@ __device__ __forceinline__ float float_up(double x)
 // when more of them come than it holds, a second scan collects them), and are skipped altogether
 // when the own surface's best ends within r1, which no triangle farther than r1 can beat; there the
 // nearest accepted triangle is usually close, and most triangles within r are never computed.
+// SPLIT lanes share a vertex: each scans every SPLIT-th group of four entries of a cell with queues and bests of
+// its own (its subset's nearest, whatever the others have), and the nearest of theirs is the vertex's. What
+// bounds the kernel: the dependent reads of a vertex's entries, in waves too few to hide them and as long as
+// their slowest lane (42,000 vertices: 321 us a lane each, 120 with four).
 // Blocks go round robin over the 8 XCDs in launch order; XCD k takes a contiguous run of vertices so
 // that neighbouring vertices, which read the same cells, share its L2.
+template <uint32_t SPLIT>
 __global__ void __launch_bounds__(kDetectBlock) __attribute__((amdgpu_waves_per_eu(3))) k_detect_bodies(contact_dev c, body_contact_dev b, const pos4* __restrict__ x)
 {
 #pragma clang fp contract(off)
@@ -326,7 +331,7 @@ __global__ void __launch_bounds__(kDetectBlock) __attribute__((amdgpu_waves_per_
     __shared__ uint32_t deferred[kDeferQueue * kDetectBlock];
     uint32_t const xcd = blockIdx.x % 8u, per = gridDim.x / 8u, extra = gridDim.x % 8u;
     uint32_t const logical = xcd * per + min(xcd, extra) + blockIdx.x / 8u;
-    uint32_t const s = logical * kDetectBlock + threadIdx.x;
+    uint32_t const s = (logical * kDetectBlock + threadIdx.x) / SPLIT, part = threadIdx.x % SPLIT;
     if (s >= c.S) return;
     uint32_t const ps = c.surf[s];
     pos4 const p = x[ps];
@@ -376,7 +381,7 @@ __global__ void __launch_bounds__(kDetectBlock) __attribute__((amdgpu_waves_per_
             src = dq, cnt = dcnt, mode = 2;
         }
         while (more && cnt <= kDetectQueue - 4) {  // scan: up to 4 entries a step, into the queue
-            if (e == n) {
+            if (e >= n) {
                 if (++cell > ncells) {
                     more = false;
                     break;
@@ -385,11 +390,11 @@ __global__ void __launch_bounds__(kDetectBlock) __attribute__((amdgpu_waves_per_
                 if (cell < ncells) {
                     ci = i0 + cell % ni, cj = j0 + (cell / ni) % nj, ck = k0 + cell / (ni * nj);
                     uint32_t const slot = hash_slot(ci, cj, ck, b.mask);
-                    e = b.start[slot], n = b.end[slot];
+                    e = b.start[slot] + 4 * part, n = b.end[slot];
                     pc[0] = float(pp[0] - double(ci) * cs), pc[1] = float(pp[1] - double(cj) * cs);
                     pc[2] = float(pp[2] - double(ck) * cs);
                 } else {
-                    e = 0, n = *b.nbig;
+                    e = part, n = *b.nbig;
                 }
                 continue;
             }
@@ -431,11 +436,12 @@ __global__ void __launch_bounds__(kDetectBlock) __attribute__((amdgpu_waves_per_
                     qu[cnt * kDetectBlock] = e + u;
                     ++cnt;
                 }
-                e += m;
+                e += 4 * SPLIT;
             } else if (mode == 1) {  // the large triangles were all computed in the first scan
                 e = n;
             } else {
-                uint32_t const t = b.big[e++];
+                uint32_t const t = b.big[e];
+                e += SPLIT;
                 pos4 const sp = b.sph[t];
                 double const ex = pp[0] - sp.x, ey = pp[1] - sp.y, ez = pp[2] - sp.z;
                 double const l = (sp.w + (t - own0 < nown ? rm : ro)) * (1.0 + 1e-9);
@@ -484,6 +490,15 @@ __global__ void __launch_bounds__(kDetectBlock) __attribute__((amdgpu_waves_per_
             }
         }
     }
+    auto nearer = [](double& d, uint32_t& t, double od, uint32_t ot) {
+        if (ot != 0xffffffffu && (t == 0xffffffffu || od < d || (od == d && ot < t))) d = od, t = ot;
+    };
+#pragma unroll
+    for (int w = 1; w < int(SPLIT); w *= 2) {
+        nearer(bo, to, __shfl_xor(bo, w, 64), uint32_t(__shfl_xor(int(to), w, 64)));
+        nearer(bm, tm, __shfl_xor(bm, w, 64), uint32_t(__shfl_xor(int(tm), w, 64)));
+    }
+    if (part) return;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {  // another body's nearest triangle, then its own surface's
         uint32_t const t = k == 0 ? to : tm;
@@ -543,7 +558,13 @@ void launch_detect_bodies(hipStream_t s, contact_dev c, body_contact_dev const& 
     uint32_t const n = uint32_t(std::size_t(kTriCells) * b.ntris);
     k_entry_records<<<grid_for(n, 256), 256, 0, s>>>(b, n);
     k_vertex_pseudonormals<<<grid_for(c.S, 256), 256, 0, s>>>(b, c.surf, x, c.S);
-    k_detect_bodies<<<grid_for(c.S, kDetectBlock), kDetectBlock, 0, s>>>(c, b, x);
+    // lanes a vertex: with more, fuller waves and shorter scans, but each lane prunes by its own best only. us a
+    // launch on 42,000 vertices of 32 bodies at rest beside each other with 1, 4, 8 and 16: 321, 120, 149, 221;
+    // a frame of folded surfaces (hundreds of entries a vertex): 4,700 vertices 2,700, 815, 474, 309; 42,000
+    // 3,008, 878, 636, 612; 415,000 12,276, 4,143, 3,919, 4,404.
+    bool const few = c.S <= 32768;
+    auto const detect = few ? k_detect_bodies<8> : k_detect_bodies<4>;
+    detect<<<grid_for(std::size_t(c.S) * (few ? 8 : 4), kDetectBlock), kDetectBlock, 0, s>>>(c, b, x);
 }
 
 void launch_body_candidates(hipStream_t s, contact_dev c, body_contact_dev const& b, const pos4* x,
