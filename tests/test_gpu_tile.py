@@ -53,6 +53,9 @@ CASES = {
     "tets_green_damped": lambda: _single(S.bar5(18, 18, 31), "green", False, beta=1e-3),
     "tets_neohookean": lambda: _single(S.ellipsoid6(0.9, 1.1, 1.4, 0.1), "neohookean", False, spheres=2),
     "tets_damped": lambda: _single(S.box6(23, 19, 17, 0.1), "neohookean", False, beta=1e-3),
+    # tiles with more than 256 elements of a color, run in two parts
+    "hex_two_chunks": lambda: _single(S.box6(280, 34, 35, 0.1), "neohookean", True, spheres=3),
+    "tets_two_chunks": lambda: _single(S.box6(110, 14, 14, 0.1), "neohookean", False, spheres=3),
     "batch_contacts": lambda: _batch(9, (6.0, 9000.0), 4),
     "batch_wide": lambda: _batch(5, (20000.0, 90000.0), 6),
 }
