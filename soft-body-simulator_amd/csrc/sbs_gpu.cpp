@@ -492,9 +492,9 @@ void sbs_gpu::color_group(group_t& g, uint32_t recolor_passes)
 // Whether the scene's frames run one workgroup per body (island.hip) instead of one launch per color:
 // every body's particles fit LDS, and the estimated time of a stage (one color of every body) is shorter.
 // A launch takes 5.1 us and 0.16 us per 1,000 hex cells (5.4 us at 2,700 cells a color, 8.2 at 20,800, 17
-// at 83,000, 82 at 445,000); a body's stage takes 3.5-4.3 us up to 256 cells (3.50 at 64, 3.82 at 128, 4.25
-// at 256), 5.4-5.8 up to 512, 7.6 up to 640, and the bodies share 256 compute units. Measured: 24x6x6 cells
-// 6.2 us a stage launched, 3.7 here; one body of 512 cells a color 5.1 launched, 5.8 here; 512 bodies of 2,900
+// at 83,000, 82 at 445,000); a body's stage takes 3.4-4.0 us up to 256 cells (3.4 at 64, 3.6 at 150; the
+// estimate is up to 0.3 above), 5.4-5.8 up to 512, 7.6 up to 640, and the bodies share 256 compute units. Measured:
+// 24x6x6 cells 6.2 us a stage launched, 3.5 here; one body of 512 cells a color 5.1 launched, 5.8 here; 512 bodies of 2,900
 // to 6,500 tets 12.3 and 5.6; 512 bodies of 8,000 to 14,000 tets 26.9 and 9.9. Green cells: 13.5-16 us
 // launched; 11.6-12.5 here up to 256 cells, 16.5 at 512. Single tets are compared with the launches that run
 // several colors in tiles, 1.3 us a stage (neo-Hookean) and 2.65 (Green) at 24,600 tets, 3.1 and 8 at 1M; here,

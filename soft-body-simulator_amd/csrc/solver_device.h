@@ -1,5 +1,5 @@
-// Device functions of the time step shared by the kernels that run one stage per launch (kernels.hip)
-// and those that run a whole frame of a small body in one launch (island.hip): position arithmetic,
+// Device functions of the time step shared by the kernels that run one stage per launch (kernels.hip), several
+// colors of a large body (tile.hip), or a whole frame of a small body (island.hip): position arithmetic,
 // prediction and velocity update, the Green, stable neo-Hookean and contact projections.
 #pragma once
 #include <type_traits>
