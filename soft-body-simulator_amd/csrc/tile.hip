@@ -566,7 +566,10 @@ void tile_scratch::build(std::vector<uint32_t> const& bounds, tile_counts const&
     uint32_t const nseg = uint32_t(bounds.size()) - 1;
     std::vector<uint4> blocks, chunks;
     std::vector<uint32_t> firsts(n.instances.size());  // [tile][color]: its first instance
-    std::size_t parts = 0, insts = 0;
+    // Instance 0 stands where a tile has no element of the segment's colors: the group's first constraints at the
+    // tile's first place, read but never run. (Any other instance's places need hold no particle in this tile,
+    // and the damping term follows a place's particle into the substep start positions.)
+    std::size_t parts = 0, insts = 1;
     plan.segments.clear();
     for (uint32_t sg = 0; sg < nseg; ++sg) {
         tile_segment seg{bounds[sg], bounds[sg + 1], 0, 0, blocks.size()};
@@ -603,6 +606,9 @@ void tile_scratch::build(std::vector<uint32_t> const& bounds, tile_counts const&
         plan.corners8.alloc(insts);
     else
         plan.corners4.alloc(insts);
+    launch_fill_u32(s, plan.elems.p, 0u, 1);
+    launch_fill_u32(s, src.hex ? reinterpret_cast<uint32_t*>(plan.corners8.p) : reinterpret_cast<uint32_t*>(plan.corners4.p),
+                    0u, src.hex ? 4 : 2);
     plan.lambda.alloc(2 * insts * per);
     plan.instances = uint32_t(insts);
     bounds_dev.upload(bounds.data(), bounds.size(), s);

@@ -35,6 +35,24 @@ def _loose_point(sc):
     return sc
 
 
+def _with_tiny_bodies(n, tets_of, kind, clusters, beta):
+    """One large body and n bodies of one cell, all in one group: a tiny body's tile has elements of one color
+    (clusters) or of six, and none in the launches of the other colors."""
+    parts = [tets_of] + [S.box6(1, 1, 1, 0.1, (0.0, 0.05, 3.0 + k)) for k in range(n)]
+    sc = scenes.Scene("tile", gravity_is_force=False, coloring="index" if clusters else "hash")
+    for x0, tets in parts:
+        s2t, tris = S.boundary(len(x0), tets)
+        sc.bodies.append(scenes.Body(x0=x0, tets=tets, mass=S.lumped_mass(x0, tets, 1000.0), surface=s2t,
+                                     triangles=tris))
+    tets = np.concatenate([t for _, t in parts])
+    sc.groups.append(scenes.Group(kind, np.repeat(np.arange(n + 1, dtype=np.uint32), [len(t) for _, t in parts]), tets,
+                                  alpha=1e-4, beta=beta, young=np.full(len(tets), 2e5),
+                                  poisson=np.full(len(tets), 0.3),
+                                  clusters=scenes.hex_clusters(len(tets)) if clusters else None))
+    sc.planes.append(((0.0, 1.0, 0.0), (0.0, 0.01, 0.0), (-1e30,) * 3, (1e30,) * 3))
+    return sc
+
+
 def _batch(n, sizes, seed):
     sc = scenes.batch(n, sizes, seed=seed, young_range=(1e4, 1e5), drop_range=(-0.01, 0.0))
     sc.body_contacts = (0.0, 0.0, 0.0)
@@ -53,6 +71,12 @@ CASES = {
     "tets_green_damped": lambda: _single(S.bar5(18, 18, 31), "green", False, beta=1e-3),
     "tets_neohookean": lambda: _single(S.ellipsoid6(0.9, 1.1, 1.4, 0.1), "neohookean", False, spheres=2),
     "tets_damped": lambda: _single(S.box6(23, 19, 17, 0.1), "neohookean", False, beta=1e-3),
+    # tiles without an element of a launch's colors: nothing of theirs reaches the damping term
+    "hex_damped_tiny": lambda: _with_tiny_bodies(5, S.box6(31, 18, 17, 0.1), "neohookean", True, 1e-3),
+    "hex_green_damped_tiny": lambda: _with_tiny_bodies(5, S.box6(23, 21, 15, 0.1), "green", True, 1e-3),
+    "tets_damped_tiny": lambda: _loose_point(_with_tiny_bodies(5, S.box6(23, 19, 17, 0.1), "neohookean", False, 1e-3)),
+    "tets_green_damped_tiny": lambda: _loose_point(_with_tiny_bodies(5, S.bar5(18, 18, 31), "green", False, 1e-3)),
+    "hex_damped_loose": lambda: _loose_point(_single(S.box6(31, 18, 17, 0.1), "neohookean", True, beta=1e-3)),
     # tiles with more than 256 elements of a color, run in two parts
     "hex_two_chunks": lambda: _single(S.box6(280, 34, 35, 0.1), "neohookean", True, spheres=3),
     "tets_two_chunks": lambda: _single(S.box6(110, 14, 14, 0.1), "neohookean", False, spheres=3),
