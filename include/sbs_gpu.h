@@ -289,6 +289,14 @@ int sbs_gpu_group_colors(sbs_gpu* sim, uint32_t group, uint32_t* num_colors, uin
  * vertex) in projection order. *count gets the total even if larger than cap. */
 int sbs_gpu_read_contacts(sbs_gpu* sim, uint32_t* ids, double* qn, uint32_t cap, uint32_t* count);
 
+/* How the frames of a committed scene are launched, chosen by sbs_gpu_commit from the sizes of the bodies and of
+ * the constraint group; the results are the same bits either way. Frames with timing on or with training rows
+ * being captured, and in tiles warm-started frames of one iteration, run one launch per color all the same. */
+#define SBS_FRAME_COLORS 0  /* one launch per color; width 0 */
+#define SBS_FRAME_TILES 1   /* several colors a launch, a workgroup per part of the particles; width: the most colors */
+#define SBS_FRAME_ISLANDS 2 /* a frame (warm-started: a substep) a launch, a workgroup per body; width: its threads */
+int sbs_gpu_frame_path(sbs_gpu* sim, int* path, uint32_t* width);
+
 /* Squared XPBD residual sum (h = C(x) + alpha~ lambda), in FP64, per color of a group, for the
  * state after the last step (dt is that step's substep length). per_color has num_colors entries. */
 int sbs_gpu_residual(sbs_gpu* sim, uint32_t group, double dt, double* per_color, uint32_t cap);

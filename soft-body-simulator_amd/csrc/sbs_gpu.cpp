@@ -2338,6 +2338,26 @@ int sbs_gpu_write_body(sbs_gpu* sim, uint32_t body, const double* x, const doubl
     });
 }
 
+int sbs_gpu_frame_path(sbs_gpu* sim, int* path, uint32_t* width)
+{
+    return guarded([&] {
+        require(sim && path && width, "null argument");
+        require(sim->committed, "sbs_gpu_commit has not been called", SBS_ERR_STATE);
+        *path = SBS_FRAME_COLORS;
+        *width = 0;
+        if (sim->islands.n) {
+            group_t const* g = nullptr;
+            for (auto const& o : sim->groups)
+                if (o.count) g = &o;
+            *path = SBS_FRAME_ISLANDS;
+            *width = island_block(g->hex, g->largest_stage);
+        } else if (sim->tiles.ready()) {
+            *path = SBS_FRAME_TILES;
+            for (auto const& s : sim->tiles.segments) *width = std::max(*width, s.last_color - s.first_color);
+        }
+    });
+}
+
 int sbs_gpu_group_colors(sbs_gpu* sim, uint32_t group, uint32_t* num_colors, uint32_t* color_of_constraint)
 {
     return guarded([&] {

@@ -97,6 +97,7 @@ _SIGS = {
     "sbs_gpu_read_body": [_p, _u32, _pd, _pd],
     "sbs_gpu_write_body": [_p, _u32, _pd, _pd],
     "sbs_gpu_group_colors": [_p, _u32, _pu, _pu],
+    "sbs_gpu_frame_path": [_p, ctypes.POINTER(_i), _pu],
     "sbs_gpu_read_contacts": [_p, _pu, _pd, _u32, _pu],
     "sbs_gpu_residual": [_p, _u32, _d, _pd, _u32],
     "sbs_gpu_energy": [_p, _pd],
@@ -589,6 +590,13 @@ class Simulation:
         c = np.zeros(self.groups[group], dtype=np.uint32)
         check(self._L.sbs_gpu_group_colors(self.h, group, ctypes.byref(nc), _up(c)))
         return c, nc.value
+
+    def frame_path(self):
+        """How the committed scene's frames are launched: "colors" (a launch per color), "tiles" or
+        "islands", and the most colors of a tile launch or the threads of an island's workgroup."""
+        path, width = _i(), _u32()
+        check(self._L.sbs_gpu_frame_path(self.h, ctypes.byref(path), ctypes.byref(width)))
+        return ("colors", "tiles", "islands")[path.value], width.value
 
     def read_contacts(self):
         cnt = _u32()

@@ -49,8 +49,7 @@ def _many(n, tets_of, kind):
 
 
 CASES = {
-    # elements of a stage: under one wave, one to four waves, colors that some bodies have no element of;
-    # hex_wide's and batch_wide's stages have more than 256 (workgroups of 512 threads)
+    # elements of a stage: under one wave, one to four waves, colors that some bodies have no element of
     "hex_small": lambda: _single(S.box6(5, 3, 4, 0.1), "neohookean", True, spheres=3),
     "hex_one_cell": lambda: _single(S.box6(1, 1, 1, 0.1), "neohookean", True),
     "hex_256": lambda: _single(S.box6(16, 16, 8, 0.1), "neohookean", True),
@@ -62,14 +61,16 @@ CASES = {
     "tets_neohookean": lambda: _single(S.ellipsoid6(0.4, 0.3, 0.5, 0.1), "neohookean", False, beta=1e-3),
     # more elements in a stage than 256 lanes
     "tets_wide": lambda: _single(S.box6(13, 13, 11, 0.1), "neohookean", False, spheres=4),
-    "tets_green_wide": lambda: _single(S.box6(12, 12, 10, 0.1), "green", False, spheres=4),
-    # the same where there are enough bodies that one workgroup each is the faster way
+    # the same of Green tets, with enough bodies that one workgroup each is the faster way
     "tets_green_wide_many": lambda: _many(45, S.box6(12, 12, 10, 0.1), "green"),
     # bodies from one cell up, boxes and ellipsoids
     "batch": lambda: scenes.batch(9, (6.0, 9000.0), seed=4, young_range=(1e4, 1e5), drop_range=(-0.01, 0.0)),
-    # up to 5,800 particles and 600 cells of a color in a body, enough bodies that it is worth it
+    # up to 4,862 particles and 540 cells of a color in a body, enough bodies that it is worth it
     "batch_wide": lambda: scenes.batch(70, (9000.0, 24000.0), seed=7, young_range=(1e4, 1e5), drop_range=(-0.01, 0.0)),
 }
+
+# threads of the workgroup where a stage of a body has more than 256 elements
+WIDE = {"tets_wide": 1024, "tets_green_wide_many": 1024, "batch_wide": 512}
 
 
 @pytest.mark.parametrize("name", sorted(CASES))
@@ -78,6 +79,7 @@ def test_island_frames_are_the_staged_frames(name, graphs):
     sc = CASES[name]()
     say(f"island {name}: {sc.num_tets} tets, {sc.num_vertices} vertices, graphs {graphs}")
     a, b = scenes.build_device(sc), scenes.build_device(sc)
+    assert a.frame_path() == ("islands", WIDE.get(name, 256))
     b.set_timing(True)
     a.use_graphs(graphs)
     rng = np.random.default_rng(8)
@@ -100,6 +102,7 @@ def test_island_iterations_after_a_warm_start(mode):
     sc = CASES["hex_256"]()
     say(f"island warm start {mode}")
     a, b = scenes.build_device(sc), scenes.build_device(sc)
+    assert a.frame_path()[0] == "islands"
     b.set_timing(True)
     nets = []
     for sim in (a, b):

@@ -72,17 +72,21 @@ CASES = {
     "tets_neohookean": lambda: _single(S.ellipsoid6(0.9, 1.1, 1.4, 0.1), "neohookean", False, spheres=2),
     "tets_damped": lambda: _single(S.box6(23, 19, 17, 0.1), "neohookean", False, beta=1e-3),
     # tiles without an element of a launch's colors: nothing of theirs reaches the damping term
-    "hex_damped_tiny": lambda: _with_tiny_bodies(5, S.box6(31, 18, 17, 0.1), "neohookean", True, 1e-3),
-    "hex_green_damped_tiny": lambda: _with_tiny_bodies(5, S.box6(23, 21, 15, 0.1), "green", True, 1e-3),
+    "hex_damped_tiny": lambda: _with_tiny_bodies(5, S.box6(130, 22, 22, 0.1), "neohookean", True, 1e-3),
+    "hex_green_damped_tiny": lambda: _loose_point(_with_tiny_bodies(5, S.box6(23, 21, 15, 0.1), "green", True, 1e-3)),
     "tets_damped_tiny": lambda: _loose_point(_with_tiny_bodies(5, S.box6(23, 19, 17, 0.1), "neohookean", False, 1e-3)),
     "tets_green_damped_tiny": lambda: _loose_point(_with_tiny_bodies(5, S.bar5(18, 18, 31), "green", False, 1e-3)),
     "hex_damped_loose": lambda: _loose_point(_single(S.box6(31, 18, 17, 0.1), "neohookean", True, beta=1e-3)),
     # tiles with more than 256 elements of a color, run in two parts
     "hex_two_chunks": lambda: _single(S.box6(280, 34, 35, 0.1), "neohookean", True, spheres=3),
     "tets_two_chunks": lambda: _single(S.box6(110, 14, 14, 0.1), "neohookean", False, spheres=3),
+    "tets_green_wide": lambda: _single(S.box6(12, 12, 10, 0.1), "green", False, spheres=4),
     "batch_contacts": lambda: _batch(9, (6.0, 9000.0), 4),
     "batch_wide": lambda: _batch(5, (20000.0, 90000.0), 6),
 }
+
+# colors a launch, where not all of a cluster group's or 7 of a tet group's
+COLORS = {"hex_one_cell": 1, "hex_thin": 4, "hex_two_chunks": 4, "batch_wide": 4, "hex_damped_tiny": 4}
 
 
 @pytest.mark.parametrize("name", sorted(CASES))
@@ -91,6 +95,7 @@ def test_tiles_are_the_staged_frames(name, graphs):
     sc = CASES[name]()
     say(f"tile {name}: {sc.num_tets} tets, {sc.num_vertices} vertices, graphs {graphs}")
     a, b = scenes.build_device(sc), scenes.build_device(sc)
+    assert a.frame_path() == ("tiles", COLORS.get(name, 8 if sc.groups[0].clusters is not None else 7))
     b.set_timing(True)
     a.use_graphs(graphs)
     rng = np.random.default_rng(8)
@@ -114,6 +119,7 @@ def test_tiles_after_a_warm_start(mode, iterations):
     sc = _single(S.box6(24, 17, 18, 0.1), "neohookean", True, spheres=4)
     say(f"tile warm start {mode}, {iterations} iterations")
     a, b = scenes.build_device(sc), scenes.build_device(sc)
+    assert a.frame_path()[0] == "tiles"
     b.set_timing(True)
     nets = []
     for sim in (a, b):
