@@ -134,3 +134,22 @@ def test_tiles_after_a_warm_start(mode, iterations):
     for got, want in zip(a.read_body(0), b.read_body(0)):
         assert np.all(np.isfinite(got)) and np.array_equal(got, want)
     a.close(), b.close()
+
+
+@pytest.mark.parametrize("mode", ["previous", "explicit"])
+@pytest.mark.parametrize("iterations", [1, 4, 5])
+def test_tiles_of_single_tets_after_a_warm_start(mode, iterations):
+    sc = CASES["tets_neohookean"]()
+    say(f"tile warm start {mode} of single tets, {iterations} iterations")
+    a, b = scenes.build_device(sc), scenes.build_device(sc)
+    assert a.frame_path() == ("tiles", 7)
+    b.set_timing(True)
+    for sim in (a, b):
+        sim.set_warm_start(mode)
+        sim.set_warm_start_scale(0.5 if mode != "explicit" else 0.2)
+        for _ in range(2):
+            sim.step(1.0 / 60.0, iterations, 4)
+    for got, want in zip(a.read_body(0), b.read_body(0)):
+        assert np.all(np.isfinite(got)) and np.array_equal(got, want)
+    assert np.array_equal(a.residual(0, 1.0 / 240.0), b.residual(0, 1.0 / 240.0))
+    a.close(), b.close()
