@@ -33,6 +33,19 @@ inline void hip_check(hipError_t e, char const* what)
     }
 }
 
+// LDS a launch may ask for without allow_lds.
+constexpr std::size_t kDefaultLds = 64 * 1024;
+
+// Raises the kernels' limit of dynamic LDS on the current device.
+template <class... Kernels>
+void allow_lds(std::size_t bytes, Kernels... kernels)
+{
+    (hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernels), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   int(bytes)),
+               "LDS limit"),
+     ...);
+}
+
 // Owning device array (hipMalloc / hipFree).
 template <class T>
 struct dev_buf {

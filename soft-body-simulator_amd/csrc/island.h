@@ -9,7 +9,10 @@ namespace sbs {
 // words.
 constexpr std::size_t kIslandLds = 160 * 1024, kIslandBytes = 28;
 constexpr uint32_t kIslandChunks = 320;
-constexpr uint32_t kIslandParticles = uint32_t((kIslandLds - 512 - 16 * kIslandChunks) / kIslandBytes);
+constexpr std::size_t kIslandDynamicLds = kIslandLds - 512;
+constexpr uint32_t kIslandParticles = uint32_t((kIslandDynamicLds - 16 * kIslandChunks) / kIslandBytes);
+constexpr std::size_t island_lds_bytes(uint32_t particles, uint32_t chunks) { return particles * kIslandBytes + chunks * 16; }
+static_assert(island_lds_bytes(kIslandParticles, kIslandChunks) <= kIslandDynamicLds, "the largest island fits");
 // Constraints of a scene of islands: 16-byte offsets into its arrays fit 32 bits.
 constexpr uint32_t kIslandConstraints = 1u << 28;
 
@@ -40,6 +43,11 @@ struct solve_params {
     float alpha_tilde, gamma;     // Green
     float inv_dt2, beta_dt;       // neo-Hookean
 };
+
+// Lets the kernels take the largest island's LDS. To be called on a device before a launch of more than
+// kDefaultLds: the limit belongs to the kernel, not to the launch, and is shared by all simulations of the
+// process, so it is always set to the same size.
+void allow_island_lds();
 
 // One launch: p.substeps substeps of every island. kind: 0 Green, 1 neo-Hookean; hex: the group's
 // elements are hex-cell clusters, else single tets.

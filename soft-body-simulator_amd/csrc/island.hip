@@ -292,21 +292,32 @@ __global__ void __launch_bounds__(BLOCK) k_island_tets(island_dev d, tet_group_d
 template <class K, class... Args>
 void launch_island(hipStream_t s, K kernel, uint32_t blocks, int block, std::size_t lds, Args... args)
 {
-    if (lds > 64 * 1024)  // more than the default limit of dynamic LDS has to be asked for
-        hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      int(lds)),
-                  "island LDS");
     kernel<<<blocks, block, lds, s>>>(args...);
 }
 
+template <int KIND, bool DAMPED>
+void allow_island_kernels()
+{
+    allow_lds(kIslandDynamicLds, k_island_hex<KIND, DAMPED, 256>, k_island_hex<KIND, DAMPED, 512>,
+              k_island_tets<KIND, DAMPED, 256>, k_island_tets<KIND, DAMPED, 1024>);
+}
+
 }  // namespace
+
+void allow_island_lds()
+{
+    allow_island_kernels<0, false>();
+    allow_island_kernels<0, true>();
+    allow_island_kernels<1, false>();
+    allow_island_kernels<1, true>();
+}
 
 void launch_island_frame(hipStream_t s, island_dev const& d, int kind, bool hex, tet_group_dev const& g,
                          cluster_dev const& cl, pos4* xi, pos4* xn, float4* v, contact_dev const& c,
                          solve_params const& p)
 {
     if (!d.count) return;
-    std::size_t const lds = std::size_t(d.cap) * kIslandBytes + std::size_t(d.chunks_cap) * 16;
+    std::size_t const lds = island_lds_bytes(d.cap, d.chunks_cap);
     bool const wide = d.block > 256, damped = kind == 0 ? p.gamma != 0.0f : p.beta_dt != 0.0f;
     auto hexes = [&](auto kernel, int block) { launch_island(s, kernel, d.count, block, lds, d, g, cl, xi, xn, v, c, p); };
     auto tets = [&](auto kernel, int block) { launch_island(s, kernel, d.count, block, lds, d, g, xi, xn, v, c, p); };

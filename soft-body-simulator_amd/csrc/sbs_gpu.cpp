@@ -973,6 +973,7 @@ void sbs_gpu::plan_islands()
     islands.upload(sorted.data(), sorted.size(), stream);
     island_chunks.upload(chunks.data(), chunks.size(), stream);
     island_list.alloc(std::max<uint32_t>(S, 1));
+    if (island_lds_bytes(largest, most) > kDefaultLds) allow_island_lds();
     hip_check(hipStreamSynchronize(stream), "upload islands");
 }
 

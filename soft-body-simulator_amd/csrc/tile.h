@@ -11,7 +11,8 @@ namespace sbs {
 // LDS bytes of a particle: its row (three coordinates and the inverse mass, FP64), the inverse mass as the
 // projections take it (FP32), its index.
 constexpr std::size_t kTileBytes = 40;
-// Particles of a tile, a multiple of 64: what a compute unit's LDS holds beside the chunks.
+// LDS of a compute unit, and the particles of a tile, a multiple of 64: what it holds beside the chunks.
+constexpr std::size_t kTileLds = 160 * 1024;
 constexpr uint32_t kTileParticles = 3968;
 // Instances of a chunk, one a lane: a wave to a SIMD. Particles are loaded and stored by twice as many threads
 // (1M tets 6,554 us for four frames, 6,728 with 256 threads).

@@ -496,12 +496,6 @@ __global__ void __launch_bounds__(kTileBlock) k_tile_emit(plan_dev d, const uint
     }
 }
 
-void allow_lds(const void* kernel, std::size_t bytes)
-{
-    if (bytes > 64 * 1024)  // more than the default limit of dynamic LDS has to be asked for
-        hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)), "tile LDS");
-}
-
 plan_dev view(tile_source const& src, dev_buf<uint32_t> const& cfirst, dev_buf<uint32_t> const& tfirst,
               dev_buf<uint32_t> const& own_first, dev_buf<uint32_t> const& own, dev_buf<uint32_t> const& tile_of,
               dev_buf<uint32_t> const& table, dev_buf<uint32_t> const& bounds, dev_buf<uint32_t> const& bits,
@@ -618,6 +612,10 @@ void tile_scratch::build(std::vector<uint32_t> const& bounds, tile_counts const&
     kernel<<<dim3(src.tiles, nseg), kTileBlock, lds, s>>>(d, plan.blocks.p, counts.p, src.surface_of, plan.particles.p,
                                                           plan.elems.p, plan.corners8.p, plan.corners4.p);
     hip_check(hipGetLastError(), "tile plan");
+    // the largest tile's LDS, whatever this plan's: the limit belongs to the kernels and is shared by all
+    // simulations of the process, so it is always set to the same size
+    allow_lds(kTileLds, k_tile_hex<0, false>, k_tile_hex<0, true>, k_tile_hex<1, false>, k_tile_hex<1, true>,
+              k_tile_tets<0, false>, k_tile_tets<0, true>, k_tile_tets<1, false>, k_tile_tets<1, true>);
     hip_check(hipStreamSynchronize(s), "tile plan");
     plan.tiles = src.tiles;
 }
@@ -632,10 +630,7 @@ void launch_tile_segment(hipStream_t s, tile_plan const& plan, std::size_t segme
                      plan.corners8.p,            plan.corners4.p, plan.lambda.p,    plan.tiles,
                      per,                        seg.cap,         plan.instances};
     std::size_t const lds = std::size_t(seg.cap) * kTileBytes + std::size_t(seg.chunks) * 16;
-    auto run = [&](auto kernel) {
-        allow_lds(reinterpret_cast<const void*>(kernel), lds);
-        kernel<<<per * kXcds, kTileThreads, lds, s>>>(d, g, in, out, xn, c, p);
-    };
+    auto run = [&](auto kernel) { kernel<<<per * kXcds, kTileThreads, lds, s>>>(d, g, in, out, xn, c, p); };
     bool const damped = kind == 0 ? p.gamma != 0.0f : p.beta_dt != 0.0f;
     if (hex && kind == 0)
         damped ? run(k_tile_hex<0, true>) : run(k_tile_hex<0, false>);
