@@ -293,6 +293,7 @@ template <class K, class... Args>
 void launch_island(hipStream_t s, K kernel, uint32_t blocks, int block, std::size_t lds, Args... args)
 {
     kernel<<<blocks, block, lds, s>>>(args...);
+    hip_check(hipGetLastError(), "island launch");
 }
 
 template <int KIND, bool DAMPED>

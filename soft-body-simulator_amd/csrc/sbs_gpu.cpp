@@ -1846,6 +1846,7 @@ void sbs_gpu::run_frame(double dt, uint32_t iterations, uint32_t substeps, int w
             hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
             try {
                 enqueue_frame(dt, iterations, substeps, warm, check);
+                hip_check(hipGetLastError(), "kernel launch");  // a graph without it would not advance the state
             } catch (...) {
                 hipGraph_t g2 = nullptr;
                 (void)hipStreamEndCapture(stream, &g2);
