@@ -47,7 +47,9 @@ struct nearest {
 // A grid node for the walk's tests: its position relative to the mesh's center in FP32, and the distance
 // `limit` beyond which nothing can be nearer than (or as near as) the best so far. The tests bound
 // distances from below in FP32; limit is the best distance widened by 1e-5 of itself and by 4e-6 of the
-// coordinates, which is several times what their roundings add up to.
+// coordinates, which is several times what their roundings add up to, and by 1e-18: a limit of which the square
+// is a normal number, beside which what is lost where squares and products are denormal does not count (a ball
+// of 1e-18 had wrong values without it). Beyond 1e19 squares are infinite, and nothing is left out.
 struct seeker {
     float x, y, z, margin, limit;
     __device__ __forceinline__ void set(mesh_dev const& mesh, const double p[3])
@@ -55,7 +57,7 @@ struct seeker {
         x = float(p[0] - mesh.center[0]);
         y = float(p[1] - mesh.center[1]);
         z = float(p[2] - mesh.center[2]);
-        margin = 4e-6f * (mesh.reach + fabsf(x) + fabsf(y) + fabsf(z));
+        margin = fmaf(4e-6f, mesh.reach + fabsf(x) + fabsf(y) + fabsf(z), 1e-18f);
         limit = INFINITY;
     }
     __device__ __forceinline__ void bound(double d2) { limit = float(sqrt(d2)) * (1.0f + 1e-5f) + margin; }
@@ -78,13 +80,14 @@ struct seeker {
         return !(box2(lo, hi) > limit * limit) && !(gap > limit);
     }
     // Whether a triangle can be: no point of it is nearer than its nearest corner along the direction to
-    // its centroid (about ten triangles a node are left for the FP64 closest point).
+    // its centroid (about ten triangles a node are left for the FP64 closest point). A square below 1e-37 counts
+    // as that: the root of a denormal is none, and nearer than 1e-18 the result is below the margin.
     __device__ __forceinline__ bool may_be(float4 a, float4 b, float4 c) const
     {
         float const ax = a.x - x, ay = a.y - y, az = a.z - z, bx = b.x - x, by = b.y - y, bz = b.z - z,
                     cx = c.x - x, cy = c.y - y, cz = c.z - z;
         float const wx = ax + bx + cx, wy = ay + by + cy, wz = az + bz + cz;
-        float const r = __builtin_amdgcn_rsqf(fmaf(wx, wx, fmaf(wy, wy, wz * wz)));
+        float const r = __builtin_amdgcn_rsqf(fmaxf(fmaf(wx, wx, fmaf(wy, wy, wz * wz)), 1e-37f));
         float const m = fminf(fminf(fmaf(ax, wx, fmaf(ay, wy, az * wz)), fmaf(bx, wx, fmaf(by, wy, bz * wz))),
                               fmaf(cx, wx, fmaf(cy, wy, cz * wz)));
         return !(m * r > limit);

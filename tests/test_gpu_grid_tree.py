@@ -1,6 +1,7 @@
 """GPU checks of the mesh-distance tree walk at its edges: triangle counts around the tree's arity and one
-level more, nodes equally far from many triangles (the ball's center, finished by a workgroup each), ties
-between equally near triangles, repeated and degenerate triangles; node values equal the oracle's."""
+level more, nodes equally far from many triangles (the ball's center), ties between equally near triangles,
+repeated and degenerate triangles, coordinates whose squares leave the FP32 range of the walk's tests; node
+values equal the oracle's."""
 import numpy as np
 import pytest
 
@@ -33,4 +34,30 @@ def test_node_values_at_the_trees_edges(mesh):
     lo, hi = V.min(0) - 0.25, V.max(0) + 0.25
     res = [4, 4, 4] if mesh == "ball" else [5, 3, 2]
     print(f"[gpu-case] grid tree {mesh}: {len(F)} triangles", flush=True)
+    assert np.array_equal(S.grid_from_mesh(V, F, lo, hi, res), O.grid_from_mesh(V, F, lo, hi, res))
+
+
+@pytest.mark.parametrize("exponent", [-45, -40, -30, *range(-23, -15), 15, 18, 19, 20, 37, 38, 39, 60])
+@pytest.mark.parametrize("shift", [0.0, 0.25])
+def test_node_values_at_any_scale(exponent, shift):
+    V, F = icosphere(0.5, 3)
+    scale = 10.0 ** exponent
+    V, lo, hi = (V + shift) * scale, (V.min(0) - 0.25) * scale, (V.max(0) + 0.25) * scale
+    print(f"[gpu-case] grid tree at scale 1e{exponent}", flush=True)
+    got, want = S.grid_from_mesh(V, F, lo, hi, [5, 4, 3]), O.grid_from_mesh(V, F, lo, hi, [5, 4, 3])
+    assert np.array_equal(got, want), (int(np.sum(got != want)), float(np.abs(got - want).max() / scale))
+
+
+@pytest.mark.parametrize("height", [0.0, 1e-19, 1e-20])
+def test_nodes_just_above_a_plate(height):
+    """Nodes above a plate at its center's height: the nearest triangle's centroid is that near to some of them."""
+    n = 24
+    i, j = np.meshgrid(np.arange(n + 1), np.arange(n + 1), indexing="ij")
+    V = np.stack([i.ravel() - n / 2, j.ravel() - n / 2, np.zeros((n + 1) ** 2)], 1).astype(np.float64)
+    a = (np.arange(n)[:, None] * (n + 1) + np.arange(n)[None, :]).ravel()
+    F = np.concatenate([np.stack([a, a + n + 1, a + 1], 1), np.stack([a + n + 1, a + n + 2, a + 1], 1)]).astype(np.uint32)
+    # the grid's nodes at thirds of the cells of the plate are its triangles' centroids
+    lo, hi = np.array([-n / 2, -n / 2, height]), np.array([n / 2, n / 2, 1.0])
+    res = [n // 2, n // 2, 2]
+    print(f"[gpu-case] grid tree {height} above a plate", flush=True)
     assert np.array_equal(S.grid_from_mesh(V, F, lo, hi, res), O.grid_from_mesh(V, F, lo, hi, res))
