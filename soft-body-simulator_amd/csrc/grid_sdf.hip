@@ -30,6 +30,7 @@ constexpr int kBlock = 256;
 constexpr uint32_t kRun = 16;  // grid nodes a wave takes (6,500 waves for 24^3 cells: six a SIMD)
 // Each of at most 16 levels leaves at most 48 children of one batch waiting while the walk goes deeper.
 constexpr uint32_t kStack = 1024, kList = 256;
+constexpr uint32_t kMaxTriangles = 1u << 30;
 
 struct grid_params {
     uint32_t res[3];
@@ -303,14 +304,25 @@ __device__ __forceinline__ float wave_min(float v)
     return v;
 }
 
+// Workgroups of k_tree_level: a wave makes one node after another, so that a level of 2^28 nodes (2^30 triangles)
+// still has fewer than 2^32 threads.
+constexpr uint32_t kMaxLevelBlocks = 1u << 20;
+constexpr uint32_t level_blocks(uint32_t nodes)
+{
+    uint32_t const blocks = (nodes + kBlock / 64 - 1) / (kBlock / 64);
+    return blocks < kMaxLevelBlocks ? blocks : kMaxLevelBlocks;
+}
+static_assert(uint64_t(kMaxLevelBlocks) * kBlock < (uint64_t(1) << 32) &&
+                  (uint64_t(kMaxTriangles) / kTreeArity + uint64_t(kMaxLevelBlocks) * (kBlock / 64)) < (uint64_t(1) << 32),
+              "threads and node indices fit 32 bits");
+
 // A wave makes a node of tree level `level`: the box of its children (triangles at level 0), and the slab that
 // holds its corners along the mean normal of its triangles, for patches of up to 256 triangles (larger ones
 // bend too far for one). sum: the nodes' summed unit normals.
-__global__ void __launch_bounds__(kBlock) k_tree_level(mesh_dev mesh, uint32_t level, float4* __restrict__ node,
-                                                       float4* __restrict__ sum)
+__device__ __forceinline__ void tree_node(mesh_dev const& mesh, uint32_t level, uint32_t i, float4* __restrict__ node,
+                                          float4* __restrict__ sum)
 {
-    uint32_t const i = (blockIdx.x * kBlock + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (i >= mesh.level_count[level]) return;
+    uint32_t const lane = threadIdx.x & 63;
     uint32_t const n = level ? mesh.level_count[level - 1] : mesh.m, below = level ? mesh.level_off[level - 1] : 0u;
     uint32_t const j0 = i * kTreeArity, have = min(kTreeArity, n - j0), j = j0 + min(lane, have - 1);
     float4 l, h, u;
@@ -369,6 +381,14 @@ __global__ void __launch_bounds__(kBlock) k_tree_level(mesh_dev mesh, uint32_t l
     }
 }
 
+__global__ void __launch_bounds__(kBlock) k_tree_level(mesh_dev mesh, uint32_t level, float4* __restrict__ node,
+                                                       float4* __restrict__ sum)
+{
+    for (uint32_t i = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); i < mesh.level_count[level];
+         i += gridDim.x * (kBlock / 64))
+        tree_node(mesh, level, i, node, sum);
+}
+
 }  // namespace
 
 // A triangle mesh on the device: its non-degenerate triangles and the tree over them, made there; then the
@@ -418,7 +438,7 @@ struct mesh_upload {
                 }
         }
         uint32_t const m = uint32_t(t.size() / 3);
-        require(m < (1u << 30), "too many triangles");
+        require(m < kMaxTriangles, "too many triangles");
         view.m = m;
         tri.upload(t.data(), t.size(), s);
         view.tri = tri.p;
@@ -451,7 +471,7 @@ struct mesh_upload {
         radix_sort_pairs(s, key.p, orig.p, m, 30, ws.p);
         k_tree_corners<<<(3 * m + 255) / 256, 256, 0, s>>>(view, position.p, corners.p, corners32.p);
         for (uint32_t l = 0; l < view.levels; ++l)
-            k_tree_level<<<(view.level_count[l] + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, s>>>(view, l, node.p, sum.p);
+            k_tree_level<<<level_blocks(view.level_count[l]), kBlock, 0, s>>>(view, l, node.p, sum.p);
         hip_check(hipGetLastError(), "mesh tree");
     }
 

@@ -61,3 +61,19 @@ def test_nodes_just_above_a_plate(height):
     res = [n // 2, n // 2, 2]
     print(f"[gpu-case] grid tree {height} above a plate", flush=True)
     assert np.array_equal(S.grid_from_mesh(V, F, lo, hi, res), O.grid_from_mesh(V, F, lo, hi, res))
+
+
+def test_more_tree_nodes_than_waves():
+    """A plate of 16.8M triangles, whose lowest tree level has more nodes than the launch that makes it has waves."""
+    n = 2900
+    assert 2 * n * n / 4 > 4 << 20
+    i, j = np.meshgrid(np.arange(n + 1), np.arange(n + 1), indexing="ij")
+    V = np.stack([i.ravel(), j.ravel(), np.zeros((n + 1) ** 2)], 1).astype(np.float64)
+    a = (np.arange(n)[:, None] * (n + 1) + np.arange(n)[None, :]).ravel()
+    F = np.concatenate([np.stack([a, a + n + 1, a + 1], 1), np.stack([a + n + 1, a + n + 2, a + 1], 1)]).astype(np.uint32)
+    lo, hi, res = np.array([1.3, 2.1, -40.0]), np.array([n - 2.7, n - 1.9, 50.0]), [17, 19, 2]
+    print(f"[gpu-case] grid tree of {len(F)} triangles", flush=True)
+    got = S.grid_from_mesh(V, F, lo, hi, res)
+    z = S.grid_node_positions(lo, hi, res)[:, 2]
+    # the nearest point lies straight below or above: coordinates of up to 2,900 round to 5e-13
+    assert np.allclose(got, z, rtol=0.0, atol=1e-10)
