@@ -199,18 +199,22 @@ extern "C" int sbs_gpu_extract_boundary(int device, uint32_t num_vertices, const
         require(num_surface_vertices && num_triangles, "size outputs are null");
         require(num_vertices <= (1u << 21), "at most 2^21 vertices");
         require(num_tets <= (1u << 28), "at most 2^28 tets");
+        // Bad indices are the caller's error whatever fails beside them, and leave the outputs alone. The device
+        // looks for them; where it cannot, the host does.
         auto check_here = [&] {
             for (std::size_t i = 0; i < 4 * std::size_t(num_tets); ++i)
                 require(tets[i] < num_vertices, "tet vertex index out of range");
+            *num_surface_vertices = *num_triangles = 0;
         };
-        *num_surface_vertices = *num_triangles = 0;
-        if (num_tets == 0) return;
-        if (hipError_t const e = hipSetDevice(device); e != hipSuccess) {
-            check_here();  // bad indices are the caller's error, with or without a device
-            hip_check(e, "hipSetDevice");
+        if (num_tets == 0) return check_here();
+        hipStream_t s = nullptr;
+        hipError_t e = hipSetDevice(device);
+        if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+        if (e != hipSuccess) {
+            check_here();
+            hip_check(e, "boundary extraction");
         }
-        hipStream_t s;
-        hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
+        bool checked = false;
         try {
             uint32_t const nf = 4 * num_tets, nv = num_vertices, fwords = (nf + 31) / 32;
             uint32_t const slots = uint32_t(nf + nf / 2 + 1);
@@ -230,7 +234,10 @@ extern "C" int sbs_gpu_extract_boundary(int device, uint32_t num_vertices, const
             launch_fill_u32(s, mem.at(o_zero), 0u, uint32_t(zeros));
             k_check_indices<<<grid_for(num_tets), 256, 0, s>>>(reinterpret_cast<const uint4*>(dt), num_tets, nv, mem.at(o_bad));
             hip_check(hipGetLastError(), "boundary face kernels");
-            require(read_word(s, mem.at(o_bad)) == 0, "tet vertex index out of range");
+            bool const bad = read_word(s, mem.at(o_bad)) != 0;
+            checked = true;
+            require(!bad, "tet vertex index out of range");
+            *num_surface_vertices = *num_triangles = 0;
             uint32_t *const bits = mem.at(o_bits), *const count = mem.at(o_count), *const before = mem.at(o_before);
             k_insert_faces<<<grid_for(nf), 256, 0, s>>>(dt, nf, slots, mem.at(o_table), mem.at(o_others), mem.at(o_least));
             k_boundary_bits<<<grid_for(nf), 256, 0, s>>>(mem.at(o_others), mem.at(o_least), nf, bits);
@@ -270,6 +277,7 @@ extern "C" int sbs_gpu_extract_boundary(int device, uint32_t num_vertices, const
             }
         } catch (...) {
             (void)hipStreamDestroy(s);
+            if (!checked) check_here();
             throw;
         }
         hip_check(hipStreamDestroy(s), "hipStreamDestroy");

@@ -1,5 +1,7 @@
 """GPU checks of the boundary extraction on meshes where faces meet in other numbers than two: the same
 surface as the host extraction, index by index."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -47,3 +49,11 @@ def test_an_index_out_of_range_is_refused():
     tets = np.arange(400, dtype=np.uint32).reshape(100, 4)
     with pytest.raises(S.SbsError, match="out of range"):
         S.extract_boundary(399, tets)
+
+
+def test_a_refused_call_leaves_its_outputs_alone():
+    tets = np.array([0, 1, 2, 3, 1, 2, 3, 9], dtype=np.uint32)
+    ns, nt = ctypes.c_uint32(77), ctypes.c_uint32(78)
+    code = S.lib().sbs_gpu_extract_boundary(0, 9, tets.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), 2, None, None,
+                                            ctypes.byref(ns), ctypes.byref(nt))
+    assert code == 1 and (ns.value, nt.value) == (77, 78)

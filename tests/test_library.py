@@ -185,3 +185,15 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True,
                        timeout=120)
     assert r.returncode == 2 and "--gpus must be 1" in r.stderr
+
+
+@pytest.mark.parametrize("device", [0, 63])
+def test_refused_boundary_extraction_leaves_its_outputs_alone(device):
+    """A bad index is the caller's error with a device, without one, and on a device that does not exist."""
+    L = S.lib()
+    tets = np.array([0, 1, 2, 3, 1, 2, 3, 9], dtype=np.uint32)
+    ns, nt = ctypes.c_uint32(77), ctypes.c_uint32(78)
+    code = L.sbs_gpu_extract_boundary(device, 9, tets.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), 2, None, None,
+                                      ctypes.byref(ns), ctypes.byref(nt))
+    assert code == 1 and b"out of range" in L.sbs_gpu_last_error()
+    assert (ns.value, nt.value) == (77, 78)
