@@ -570,7 +570,10 @@ void sbs_gpu::upload_group(group_t& g)
     bool const by_body = small_bodies(g);
     if (by_body) {
         // body by body inside each color (a body's elements are then one run of it); elements of
-        // one color are independent, so their order does not change the result
+        // one color are independent, so their order does not change the result. Clusters of other
+        // shapes than hex cells, which no island runs, take this order too: their launches have no use
+        // for the regions below, which only scatter a color's clusters (512 bodies of 7,865 tets in
+        // clusters of five, 16 sweeps: 3,320 us a frame so, 3,577 by regions; 256 bodies 1,738 and 1,889)
         for (uint32_t c = 0; c < g.ncolors; ++c)
             std::stable_sort(eorder.begin() + g.cluster_color_offsets[c], eorder.begin() + g.cluster_color_offsets[c + 1],
                              [&](uint32_t a, uint32_t b) { return g.body_of(e_begin(a)) < g.body_of(e_begin(b)); });
