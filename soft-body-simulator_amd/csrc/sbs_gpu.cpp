@@ -1116,7 +1116,7 @@ void sbs_gpu::plan_tiles(std::vector<pos4> const& x)
         tile_source const src{V, g->num_elements(), g->ncolors, g->hex, g->hex ? g->cl_v0.p : g->idx.p, g->cl_v1.p,
                               first.data(), g->color_offsets.data(), surface_of_dev.p, tile_of.data(), n};
         tile_scratch scratch(stream, src);
-        for (uint32_t per : {8u, 4u, 2u}) {
+        for (uint32_t per : {kTileColors, 4u, 2u}) {
             uint32_t const nseg = (g->ncolors + per - 1) / per;
             std::vector<uint32_t> b(nseg + 1);
             for (uint32_t k = 0; k <= nseg; ++k) b[k] = uint32_t(uint64_t(g->ncolors) * k / nseg);

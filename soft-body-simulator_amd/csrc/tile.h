@@ -17,6 +17,9 @@ constexpr uint32_t kTileParticles = 3968;
 // Instances of a chunk, one a lane: a wave to a SIMD. Particles are loaded and stored by twice as many threads
 // (1M tets 6,554 us for four frames, 6,728 with 256 threads).
 constexpr int kTileBlock = 256, kTileThreads = 512;
+// Colors of a launch, and chunks of a tile in one: elements of a color share no particle.
+constexpr uint32_t kTileColors = 8, kTileChunks = kTileColors * ((kTileParticles + kTileBlock - 1) / kTileBlock);
+static_assert(kTileParticles * kTileBytes + kTileChunks * 16 <= kTileLds, "the largest tile fits");
 // Constraints of a scene of tiles: 16-byte offsets into its arrays fit 32 bits.
 constexpr uint32_t kTileConstraints = 1u << 28;
 // Largest scratch memory of the plan.
@@ -68,7 +71,7 @@ struct tile_counts {
 };
 
 // Plans in two steps: tile_scratch::count() for candidate segmentations, build() for the chosen one.
-struct tile_scratch {
+struct tile_scratch {  // (build() throws SBS_ERR_OUT_OF_MEMORY for a plan that is too large as well)
     tile_scratch(hipStream_t s, tile_source const& src);
     // (all particles ~0u: the plan would take more scratch memory than kTileScratch)
     tile_counts count(std::vector<uint32_t> const& bounds);  // bounds: first color of each segment, then ncolors

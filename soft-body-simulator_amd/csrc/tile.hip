@@ -136,6 +136,9 @@ __device__ __forceinline__ void run_tile(tile_dev const& d, const pos4* __restri
     load_rows(0);
     if (runs) data(first);
     loads_issued();
+    // (a tile holds at most one batch of particles and kTileThreads words of chunks: the loops below never turn.
+    // Without them the compiler schedules the loads above otherwise, and four frames of 1M tets take 6,664 us
+    // instead of 6,533, two of 129k 2,250 instead of 2,228)
     if (tid < 4 * n) P.chunk[tid] = rec;
     for (uint32_t k = tid + kTileThreads; k < 4 * n; k += kTileThreads) P.chunk[k] = recs[k];
     put_rows(0);
@@ -590,7 +593,9 @@ void tile_scratch::build(std::vector<uint32_t> const& bounds, tile_counts const&
         plan.segments.push_back(seg);
     }
     int const per = src.hex ? kHexTets : 1;
-    require(parts < (std::size_t(1) << 31) && insts * per < (std::size_t(1) << 29), "tile plan too large");
+    // offsets of 32 bits; as with a plan that memory has no room for, the caller does without
+    require(parts < (std::size_t(1) << 31) && insts * per < (std::size_t(1) << 29), "tile plan too large",
+            SBS_ERR_OUT_OF_MEMORY);
     plan.blocks.upload(blocks.data(), blocks.size(), s);
     plan.chunks.upload(chunks.data(), chunks.size(), s);
     counts.upload(firsts.data(), firsts.size(), s);
