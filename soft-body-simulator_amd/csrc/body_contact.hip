@@ -561,7 +561,11 @@ void launch_detect_bodies(hipStream_t s, contact_dev c, body_contact_dev const& 
     // lanes a vertex: with more, fuller waves and shorter scans, but each lane prunes by its own best only. us a
     // launch on 42,000 vertices of 32 bodies at rest beside each other with 1, 4, 8 and 16: 321, 120, 149, 221;
     // a frame of folded surfaces (hundreds of entries a vertex): 4,700 vertices 2,700, 815, 474, 309; 42,000
-    // 3,008, 878, 636, 612; 415,000 12,276, 4,143, 3,919, 4,404.
+    // 3,008, 878, 636, 612; 415,000 12,276, 4,143, 3,919, 4,404. The whole detection of bodies that keep their
+    // shapes, with 4 and 8: 2,510 vertices 95 and 82, 9,400 120 and 104, 22,800 115 and 103, 30,200 118 and 130,
+    // 62,000 172 and 179, 426,000 727 and 878; as they begin to fold (16 frames on): 9,400 208 and 143, 30,200 189
+    // and 150, 62,000 284 and 246, 426,000 945 and 1,031. So 4 where the shapes are kept and the vertices are
+    // many, 8 below; about 30,000 either gains less than folding costs.
     bool const few = c.S <= 32768;
     auto const detect = few ? k_detect_bodies<8> : k_detect_bodies<4>;
     detect<<<grid_for(std::size_t(c.S) * (few ? 8 : 4), kDetectBlock), kDetectBlock, 0, s>>>(c, b, x);
