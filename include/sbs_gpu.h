@@ -247,7 +247,9 @@ int sbs_gpu_set_coloring(sbs_gpu* sim, int order);
 /* Threads per block of the per-constraint kernels (64/128/256) and of the cluster kernels
  * (64/128, or SBS_CLUSTER_BLOCK_STREAMED: 64 threads, and the neo-Hookean hex-cell kernel loads
  * each tet's material just before projecting it instead of all six up front -- fewer registers,
- * more waves in flight, for launches large enough to be bandwidth bound). Default 256 and 64. */
+ * more waves in flight, for launches large enough to be bandwidth bound). Default 256 and 64.
+ * Frames in tiles (sbs_gpu_frame_path) use the first for their prediction and velocity update only and
+ * the second not at all, frames in islands neither. */
 #define SBS_CLUSTER_BLOCK_STREAMED 65
 int sbs_gpu_set_launch_config(sbs_gpu* sim, int block, int cluster_block);
 /* Default on (no reference counterpart): when the scene's only constraint group is neo-Hookean

@@ -72,7 +72,15 @@ STREAMED = 65  # SBS_CLUSTER_BLOCK_STREAMED
 
 
 def tune_launch(sim, scene, frames=5, blocks=(128, 256), cluster_blocks=(64, 128, STREAMED)):
-    """Fastest (block, cluster_block) over a few graph-replayed frames; leaves it set."""
+    """Fastest (block, cluster_block) over a few graph-replayed frames; leaves it set. What the scene's
+    frames do not use (frame_path) is not swept: tiles have no use for cluster_block, islands for neither;
+    the launches per color that such a scene runs with timing on then take 256 and 64, the defaults, where
+    those are among the candidates."""
+    path, _ = sim.frame_path()
+    if path != "colors":
+        cluster_blocks = (64,) if 64 in cluster_blocks else cluster_blocks[:1]
+    if path == "islands":
+        blocks = (256,) if 256 in blocks else blocks[:1]
     best = None
     sim.snapshot()
     for b in blocks:
