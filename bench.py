@@ -19,7 +19,9 @@ the scale the tuner found best for that count on the tuning frames).
 solver's.
 
 After the timed regions an instrumented region (HIP events around every launch on the library's
-stream) measures the average duration of the tet projection kernel for the roofline figure. The
+stream) measures the average duration of the tet projection kernel for the roofline figure. Those
+frames launch one color at a time; how the timed ones are launched, and their whole time against the
+same bytes, stands beside it (config.frames, roofline.timed_plain_frames). The
 CPU baseline times the FP64 oracle in the reference's insertion order on one pinned core over a
 bounded sample (5 frames after 5 warm-up frames of the same scene, or of a 16-body batch scaled by
 tet count for the batches); the accuracy legs compare the device with the oracle from rest.
@@ -43,6 +45,16 @@ BYTES_PER_TET = 184
 
 def log(msg):
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
+
+
+def frame_launches(sim, scene):
+    """How the scene's frames are launched, and the kernel that projects the tets in them. (Frames with timing on
+    launch color by color whatever this says: the instrumented region's projection kernel.)"""
+    path, width = sim.frame_path()
+    shape = ("_hex" if scene.groups[0].clusters is not None else "") if path == "colors" else (
+        "_hex" if scene.groups[0].clusters is not None else "_tets")
+    kernel = {"colors": f"k_{scene.groups[0].kind}", "tiles": "k_tile", "islands": "k_island"}[path] + shape
+    return {"path": path, "width": width, "projection_kernel": kernel}
 
 
 def cpu_model():
@@ -411,7 +423,8 @@ def main():
     t0 = time.perf_counter()
     sim = scenes.build_device(scene)
     _, ncolors = sim.group_colors(0)
-    log(f"committed in {time.perf_counter() - t0:.1f}s, {ncolors} colors")
+    frames = frame_launches(sim, scene)
+    log(f"committed in {time.perf_counter() - t0:.1f}s, {ncolors} colors, frames {frames}")
     kind = {"green": S._lib.KERNEL_GREEN, "neohookean": S._lib.KERNEL_NEOHOOKEAN}[scene.groups[0].kind]
     warmable = scene.groups[0].kind == "neohookean" and not args.no_learned
     if warmable and scene.body_contacts is not None:
@@ -573,6 +586,9 @@ def main():
     achieved = bytes_per_launch / avg_launch_s / 1e9
     log(f"projection kernel: {launches} launches, avg {1e6 * avg_launch_s:.2f} us, {units / launches:.0f} tets/launch, "
         f"{achieved:.1f} GB/s algorithmic")
+    # the timed plain frames as a whole (every kernel of theirs) against the same bytes
+    sweep_s = 1.0 / (plain_sps * scene.iterations)
+    sweep_gbs = BYTES_PER_TET * scene.num_tets / sweep_s / 1e9
     res = float(sum(sim.residual(0, scene.dt / scene.substeps)) ** 0.5)
     sim.close()
 
@@ -644,6 +660,7 @@ def main():
             "launch_config": launch,
             "obstacles": f"ground plane + {len(scene.spheres)} spheres",
             "launch": "hipGraph per frame",
+            "frames": frames,
             "parallelism": "single GPU",
             "positions": "fp64 storage, fp32 constraint arithmetic, fp64 residual norms",
         },
@@ -677,6 +694,10 @@ def main():
             "bytes_per_unit": BYTES_PER_TET,
             "units_per_launch": round(units / launches, 1),
             "avg_launch_us": round(1e6 * avg_launch_s, 3),
+            "measured_on": "frames with timing on, one launch per color",
+            "timed_plain_frames": {"projection_kernel": frames["projection_kernel"],
+                                   "us_per_iteration": round(1e6 * sweep_s, 3), "achieved": round(sweep_gbs, 2),
+                                   "frac": round(sweep_gbs / HBM_PEAK_GBS, 4)},
         },
         "kernels": per_kernel,
         "other_workloads": others or None,
@@ -733,6 +754,7 @@ def plain_throughput(scene, kind, args, warmup=3, frames=5, reps=3):
     sim = scenes.build_device(scene)
     build = time.perf_counter() - t0
     sim.use_graphs(True)
+    launches_of_frames = frame_launches(sim, scene)
     launch = autotune.tune_launch(sim, scene, frames=2)
     for _ in range(warmup):
         sim.step(scene.dt, scene.iterations, scene.substeps)
@@ -762,13 +784,15 @@ def plain_throughput(scene, kind, args, warmup=3, frames=5, reps=3):
                          "contacts_with_own_surface": int(len(t)) - other,
                          "contacts_with_obstacles": int(len(ids) - len(t))}
     sim.close()
+    sweep_gbs = BYTES_PER_TET * scene.num_tets * scene.iterations * scene.substeps * frames / med / 1e9
     avg = ms / 1e3 / launches
     gbs = BYTES_PER_TET * units / launches / avg / 1e9
     sps = frames * scene.substeps / med
     log(f"{scene.name}: plain {sps:.1f} substeps/s, projection {1e6 * avg:.2f} us per launch ({gbs:.0f} GB/s), "
         f"built in {build:.1f}s")
     return {"workload": scene.name, "tets": scene.num_tets, "plain_substeps_per_s": round(sps, 2),
-            "launch_config": launch, "projection_avg_launch_us": round(1e6 * avg, 3),
+            "launch_config": launch, "frames_launched_as": launches_of_frames,
+            "timed_frames_GBps": round(sweep_gbs, 1), "projection_avg_launch_us": round(1e6 * avg, 3),
             "roofline_frac": round(gbs / HBM_PEAK_GBS, 4), "achieved_GBps": round(gbs, 1),
             "contact_overflow": overflow, "frames": f"median of {reps} x {frames} frames after {warmup}",
             "detect_ms_per_frame": round(detect_ms, 3),
