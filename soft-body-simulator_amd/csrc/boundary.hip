@@ -10,7 +10,7 @@
 // vertex orders; surface vertices are numbered by first appearance along the boundary triangles. Both orders
 // are bits set at indices and the bits' prefix sums, so nothing is sorted.
 //
-// What bounds it: at 1M tets (4M faces, 1.53 ms a call) the upload of 16 MB from the caller's memory, 0.9 ms;
+// What bounds it: at 1M tets (4M faces, 1.65 ms a call) the upload of 16 MB from the caller's memory, 0.9 ms;
 // then the insertion's random accesses, an atomic on the table and a look at another tet for each face, 279 us
 // of 430 on the device. Sorting the faces by their keys moved them through seven radix passes, 149 launches
 // and 860 us; its 18 buffers took 2.6 ms of a call of 4.5 to allocate and free, the two here 0.4.

@@ -1,4 +1,4 @@
-// Whole-frame kernels of small bodies (island.hip): one workgroup per island.
+// Whole-frame kernels of small bodies (island.hip): one workgroup per island (body).
 #pragma once
 #include "kernels.h"
 

@@ -1,5 +1,5 @@
-// A whole frame of small bodies in one launch: one workgroup per island (a body, or bodies joined by
-// constraints) keeps the island's working positions in LDS and runs prediction, every iteration's
+// A whole frame of small bodies in one launch: one workgroup per island (a body that no constraint joins to
+// another) keeps the island's working positions in LDS and runs prediction, every iteration's
 // contacts and colors, and the velocity update with a workgroup barrier between stages, instead of
 // one launch per stage.
 //
