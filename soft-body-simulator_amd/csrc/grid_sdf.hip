@@ -9,7 +9,8 @@
 // sum of incident face normals weighted by the incident angles, the edge normal sum of the normals
 // of the faces sharing the edge, or the face normal. Zero-area triangles are left out.
 //
-// A wave per grid node walks a tree of bounds over the triangles in Morton order (k_grid_nodes). What bounds
+// A wave per grid node walks a tree of bounds over the triangles in Morton order (k_grid_nodes); up to 512
+// triangles are scanned instead (k_grid_scan). What bounds
 // it: the FP32 tests of a few hundred tree nodes and triangles a grid node and the round trips to L2 between
 // the batches. On the 20,480-triangle ball and 24^3 cells (104,625 nodes) 963 us, where the scan of
 // 128-triangle tiles through LDS that it replaces took 12.4 ms.
@@ -31,6 +32,9 @@ constexpr uint32_t kRun = 16;  // grid nodes a wave takes (6,500 waves for 24^3 
 // Each of at most 16 levels leaves at most 48 children of one batch waiting while the walk goes deeper.
 constexpr uint32_t kStack = 1024, kList = 256;
 constexpr uint32_t kMaxTriangles = 1u << 30;
+// Meshes that are scanned instead, and grids whose nodes take eight lanes each in the scan (k_grid_scan).
+constexpr uint32_t kScanTriangles = 512;
+constexpr uint64_t kSplitNodes = 131072;
 
 struct grid_params {
     uint32_t res[3];
@@ -95,7 +99,8 @@ struct seeker {
     }
 };
 
-// Triangle t's exact closest point against the best so far.
+// Triangle t's exact closest point against the best so far. MORTON: t counts in Morton order, not in their own.
+template <bool MORTON>
 __device__ __forceinline__ void visit(mesh_dev const& mesh, uint32_t t, const double p[3], nearest& best)
 {
 #pragma clang fp contract(off)
@@ -105,22 +110,22 @@ __device__ __forceinline__ void visit(mesh_dev const& mesh, uint32_t t, const do
     tri_closest_point(p, c, q, &feat);
     double const e0 = p[0] - q[0], e1 = p[1] - q[1], e2 = p[2] - q[2];
     double const d2 = e0 * e0 + e1 * e1 + e2 * e2;
-    uint32_t const o = mesh.orig[t];
+    uint32_t const o = MORTON ? mesh.orig[t] : t;
     if (d2 < best.d2 || (d2 == best.d2 && o < best.o)) best = nearest{d2, t, o};
 }
 
-// Every lane gets the nearest of the wave's.
-__device__ __forceinline__ void wave_nearest(nearest& best)
+// Every lane gets the nearest of its `lanes` neighbours.
+__device__ __forceinline__ void wave_nearest(nearest& best, int lanes = 64)
 {
-    for (int o = 32; o > 0; o >>= 1) {
+    for (int o = lanes / 2; o > 0; o >>= 1) {
         nearest const b{__shfl_xor(best.d2, o, 64), uint32_t(__shfl_xor(best.t, o, 64)), uint32_t(__shfl_xor(best.o, o, 64))};
         if (b.d2 < best.d2 || (b.d2 == best.d2 && b.o < best.o)) best = b;
     }
 }
 
-// The signed distance from the nearest triangle t (in Morton order): its closest point again, the
-// pseudo-normal of the feature that holds it (an edge's is the sum of its triangles' unit normals in original
-// order).
+// The signed distance from the nearest triangle t: its closest point again, the pseudo-normal of the feature
+// that holds it (an edge's is the sum of its triangles' unit normals in original order).
+template <bool MORTON>
 __device__ __forceinline__ double signed_distance(mesh_dev const& mesh, mesh_normals const& nm, const double p[3],
                                                   uint32_t t)
 {
@@ -128,7 +133,7 @@ __device__ __forceinline__ double signed_distance(mesh_dev const& mesh, mesh_nor
     if (t == 0xffffffffu) return DBL_MAX;
     double c[9], q[3], nrm[3] = {0.0, 0.0, 0.0};
     for (int k = 0; k < 9; ++k) c[k] = mesh.corners[9 * std::size_t(t) + k];
-    uint32_t const o = mesh.orig[t];
+    uint32_t const o = MORTON ? mesh.orig[t] : t;
     int feat;
     tri_closest_point(p, c, q, &feat);
     const uint32_t* tv = mesh.tri + 3 * std::size_t(o);
@@ -167,15 +172,13 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
     uint64_t const l0 = (uint64_t(blockIdx.x) * kWaves + wave) * kRun;
     if (l0 >= n) return;
     uint32_t const cnt = uint32_t(n - l0 < kRun ? n - l0 : kRun);
-    if (mesh.m == 0) {
-        if (lane < cnt) out[l0 + lane] = 0xffffffffu;
-        return;
-    }
     uint32_t* const stack = stack_lds[wave];
     uint32_t* const list = list_lds[wave];
     uint64_t const below = (uint64_t(1) << lane) - 1;
     grid_dims const dims(gp.res);
-    uint32_t const top = mesh.levels - 1, start = top < 2 ? top : 2;
+    static_assert(kScanTriangles >= 64, "a tree has three levels at least");
+    uint32_t const top = mesh.levels - 1;
+    constexpr uint32_t start = 2;
     uint32_t mine = 0xffffffffu;  // lane r: the nearest of node l0 + r
     uint32_t block = 0;  // of 64 triangles
     for (uint32_t r = 0; r < cnt; ++r) {
@@ -183,7 +186,7 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
         grid_node_position(dims, gp.dmin, gp.cell, l0 + r, p);
         seeker at;
         at.set(mesh, p);
-        if (r == 0 && top >= 2) {  // a node two levels up is one block of 64 triangles
+        if (r == 0) {  // a node two levels up is one block of 64 triangles
             float md = INFINITY;
             for (uint32_t i = lane; i < mesh.level_count[start]; i += 64) {
                 const float4* node = mesh.node + 3 * (std::size_t(mesh.level_off[start]) + i);
@@ -197,7 +200,7 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
             }
         }
         nearest best;
-        if (64 * block + lane < mesh.m) visit(mesh, 64 * block + lane, p, best);
+        if (64 * block + lane < mesh.m) visit<true>(mesh, 64 * block + lane, p, best);
         wave_nearest(best);
         at.bound(best.d2);
         uint32_t sp = 0, candidates = 0;
@@ -208,7 +211,7 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
             __builtin_amdgcn_wave_barrier();
         };
         auto drain = [&] {
-            for (uint32_t i = lane; i < candidates; i += 64) visit(mesh, list[i], p, best);
+            for (uint32_t i = lane; i < candidates; i += 64) visit<true>(mesh, list[i], p, best);
             candidates = 0;
             __builtin_amdgcn_wave_barrier();
         };
@@ -246,6 +249,39 @@ __global__ void __launch_bounds__(kBlock) k_grid_nodes(mesh_dev mesh, grid_param
     if (lane < cnt) out[l0 + lane] = mine;
 }
 
+// A mesh of few triangles, in their own order: SPLIT lanes take a grid node, each scans every SPLIT-th triangle, with
+// the walk's FP32 test before an exact closest point, and the nearest of theirs is the node's. With one lane the
+// triangles' reads are the wave's, through the scalar cache. What bounds it: the chain of exact closest points a
+// lane computes in grids of few nodes, the arithmetic of all lanes in large ones. A call in us, scanned and with
+// the tree (whose making alone is 25 launches, and whose walk keeps a wave busy a node): 12 triangles and 24^3
+// cells 205 and 410, 40^3 460 and 1,010, 64^3 1,330 and 3,330; a ball of 320 triangles and 12^3 cells 195 and 380 to
+// 520, 24^3 295 and 500, 40^3 670 and 1,280. A ball of 1,280: 24^3 515 and 565, 64^3 3,260 and 4,745; a double cone of
+// 400: 24^3 420 and 595, 40^3 1,220 and 1,410; of 800: 655 and 750, but 1,980 and 1,630; a ball of 5,120: 1,310 and
+// 840. So 512 triangles, below which the scan is never the slower one. Eight lanes a node or one: a ball of 320
+// triangles, 12^3 cells 195 and 315, 24^3 (105,000 nodes) 295 and 335, 40^3 (472,000) 800 and 670; a double cone of 400,
+// 420 and 590, then 1,160 and 1,220; 64^3 (1.9M) 4,350 and 3,230.
+template <uint32_t SPLIT>
+__global__ void __launch_bounds__(kBlock) k_grid_scan(mesh_dev mesh, mesh_normals nm, grid_params gp, uint64_t n,
+                                                      double* __restrict__ out)
+{
+    uint64_t const l = (uint64_t(blockIdx.x) * kBlock + threadIdx.x) / SPLIT;
+    if (l >= n) return;
+    double p[3];
+    grid_node_position(grid_dims(gp.res), gp.dmin, gp.cell, l, p);
+    seeker at;
+    at.set(mesh, p);
+    nearest best;
+    for (uint32_t t = SPLIT == 1 ? 0u : threadIdx.x % SPLIT; t < mesh.m; t += SPLIT) {
+        const float4* c = mesh.corners32 + 3 * std::size_t(t);
+        if (!at.may_be(c[0], c[1], c[2])) continue;
+        double const before = best.d2;
+        visit<false>(mesh, t, p, best);
+        if (best.d2 < before) at.bound(best.d2);
+    }
+    wave_nearest(best, int(SPLIT));
+    if (threadIdx.x % SPLIT == 0) out[l] = signed_distance<false>(mesh, nm, p, best.t);
+}
+
 __global__ void __launch_bounds__(kBlock) k_grid_signs(mesh_dev mesh, mesh_normals nm, grid_params gp, uint64_t n,
                                                        const uint32_t* __restrict__ nearest_of, double* __restrict__ out)
 {
@@ -253,7 +289,7 @@ __global__ void __launch_bounds__(kBlock) k_grid_signs(mesh_dev mesh, mesh_norma
     if (l >= n) return;
     double p[3];
     grid_node_position(grid_dims(gp.res), gp.dmin, gp.cell, l, p);
-    out[l] = signed_distance(mesh, nm, p, nearest_of[l]);
+    out[l] = signed_distance<true>(mesh, nm, p, nearest_of[l]);
 }
 
 // ---------------------------------------------------------------- the tree
@@ -391,8 +427,8 @@ __global__ void __launch_bounds__(kBlock) k_tree_level(mesh_dev mesh, uint32_t l
 
 }  // namespace
 
-// A triangle mesh on the device: its non-degenerate triangles and the tree over them, made there; then the
-// normals that give the distance its sign, made on the host (FP64, no FMA contraction) while the device walks
+// A triangle mesh on the device: its non-degenerate triangles and, where there are more than a scan takes, the
+// tree over them, made there; then the normals that give the distance its sign, made on the host (FP64, no FMA contraction) while the device walks
 // the tree. (The tree made on the host, and everything before the walk: 3.57 ms for the 20,480-triangle ball and
 // 24^3 cells, 1.53 ms so, 0.93 of it the walk.)
 struct mesh_upload {
@@ -443,13 +479,16 @@ struct mesh_upload {
         tri.upload(t.data(), t.size(), s);
         view.tri = tri.p;
         if (!m) return;
+        if (m <= kScanTriangles) {
+            upload_corners(s, pos, lo, hi);
+            return;
+        }
         morton_box box;
         for (int d = 0; d < 3; ++d) {
             box.lo[d] = lo[d];
             box.scale[d] = hi[d] > lo[d] ? 1024.0 / (hi[d] - lo[d]) : 0.0;
-            view.center[d] = 0.5 * (lo[d] + hi[d]);
-            view.reach = std::max(view.reach, float(0.5 * (hi[d] - lo[d])) * (1.0f + 1e-6f));
         }
+        center(lo, hi);
         uint32_t nodes = 0;
         for (uint32_t n = m; view.levels < kTreeLevels;) {
             n = (n + kTreeArity - 1) / kTreeArity;
@@ -475,7 +514,33 @@ struct mesh_upload {
         hip_check(hipGetLastError(), "mesh tree");
     }
 
-    // The normals' host arrays stay until the stream has taken them.
+    // The corners alone, in the triangles' own order, for k_grid_scan: FP64 and then relative to the center in FP32.
+    void upload_corners(hipStream_t s, const double* pos, const double lo[3], const double hi[3])
+    {
+        center(lo, hi);
+        std::size_t const n = 3 * std::size_t(view.m), first32 = (3 * n + 1) & ~std::size_t(1);
+        host_corners.resize(first32 + 2 * n);
+        auto* const c32 = reinterpret_cast<float4*>(host_corners.data() + first32);
+        for (std::size_t i = 0; i < n; ++i) {
+            const double* x = pos + 3 * std::size_t(t[i]);
+            std::copy(x, x + 3, host_corners.data() + 3 * i);
+            c32[i] = make_float4(float(x[0] - view.center[0]), float(x[1] - view.center[1]), float(x[2] - view.center[2]),
+                                 0.0f);
+        }
+        corners.upload(host_corners.data(), host_corners.size(), s);
+        view.corners = corners.p, view.corners32 = reinterpret_cast<const float4*>(corners.p + first32);
+    }
+
+    void center(const double lo[3], const double hi[3])
+    {
+        for (int d = 0; d < 3; ++d) {
+            view.center[d] = 0.5 * (lo[d] + hi[d]);
+            view.reach = std::max(view.reach, float(0.5 * (hi[d] - lo[d])) * (1.0f + 1e-6f));
+        }
+    }
+
+    // The host arrays stay until the stream has taken them.
+    std::vector<double> host_corners;
     std::vector<double> vn, fn;
     std::vector<uint32_t> off, inc;
 
@@ -562,9 +627,18 @@ void build_mesh_grid(hipStream_t s, const double* pos, uint32_t nv, const uint32
         gp.dmin[d] = dmin[d];
     }
     uint64_t const n = grid_dims(res).nodes(), per_block = uint64_t(kRun) * (kBlock / 64);
-    dev_buf<uint32_t> nearest_of;
-    nearest_of.alloc(n);
     mesh_upload mesh(s, pos, nv, tris, nt);
+    dev_buf<uint32_t> nearest_of;
+    if (mesh.view.m <= kScanTriangles) {
+        mesh_normals const nm = mesh.normals(s, pos, nv);
+        uint32_t const split = n <= kSplitNodes ? 8u : 1u;
+        auto const scan = split > 1 ? k_grid_scan<8> : k_grid_scan<1>;
+        scan<<<unsigned((n * split + kBlock - 1) / kBlock), kBlock, 0, s>>>(mesh.view, nm, gp, n, dev_nodes);
+        hip_check(hipGetLastError(), "grid node kernel");
+        hip_check(hipStreamSynchronize(s), "grid node kernel");
+        return;
+    }
+    nearest_of.alloc(n);
     k_grid_nodes<<<unsigned((n + per_block - 1) / per_block), kBlock, 0, s>>>(mesh.view, gp, n, nearest_of.p);
     hip_check(hipGetLastError(), "grid node kernel");
     mesh_normals const nm = mesh.normals(s, pos, nv);

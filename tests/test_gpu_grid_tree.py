@@ -1,4 +1,4 @@
-"""GPU checks of the mesh-distance tree walk at its edges: triangle counts around the tree's arity and one
+"""GPU checks of the mesh-distance scan and tree walk at their edges: triangle counts around the tree's arity and one
 level more, nodes equally far from many triangles (the ball's center), ties between equally near triangles,
 repeated and degenerate triangles, coordinates whose squares leave the FP32 range of the walk's tests; node
 values equal the oracle's."""
@@ -37,10 +37,36 @@ def test_node_values_at_the_trees_edges(mesh):
     assert np.array_equal(S.grid_from_mesh(V, F, lo, hi, res), O.grid_from_mesh(V, F, lo, hi, res))
 
 
+@pytest.mark.parametrize("triangles", [511, 512, 513, 1024, 1025, 4096, 4097])
+def test_node_values_where_the_tree_begins(triangles):
+    """Up to 512 triangles are scanned, more walked; trees of one node more and fewer on a level."""
+    V, F = _strip(triangles)
+    lo, hi = V.min(0) - 0.25, V.max(0) + 0.25
+    print(f"[gpu-case] grid of {triangles} triangles", flush=True)
+    assert np.array_equal(S.grid_from_mesh(V, F, lo, hi, [31, 3, 2]), O.grid_from_mesh(V, F, lo, hi, [31, 3, 2]))
+
+
+@pytest.mark.parametrize("mesh", ["strip_1", "strip_7", "strip_9", "messy", "fan"])
+@pytest.mark.parametrize("res", [(1, 1, 1), (25, 25, 25), (26, 26, 26)])
+def test_scanned_meshes_with_eight_lanes_a_node_and_one(mesh, res):
+    """Grids of up to 131,072 nodes (25^3 cells have 118,976, 26^3 133,407) take eight lanes a node."""
+    if mesh == "fan":
+        a = 2 * np.pi * np.arange(150) / 150
+        V = np.concatenate([[[0.0, 0.0, 1.0], [0.0, 0.0, -1.0]], np.stack([np.cos(a), np.sin(a), 0 * a], 1)])
+        i, j = 2 + np.arange(150), 2 + (np.arange(150) + 1) % 150
+        F = np.concatenate([np.stack([0 * i, i, j], 1), np.stack([0 * i + 1, j, i], 1)]).astype(np.uint32)
+    else:
+        V, F = _messy() if mesh == "messy" else _strip(int(mesh[6:]))
+    lo, hi = V.min(0) - 0.25, V.max(0) + 0.25
+    print(f"[gpu-case] scanned grid {mesh} {res}", flush=True)
+    assert np.array_equal(S.grid_from_mesh(V, F, lo, hi, list(res)), O.grid_from_mesh(V, F, lo, hi, list(res)))
+
+
 @pytest.mark.parametrize("exponent", [-45, -40, -30, *range(-23, -15), 15, 18, 19, 20, 37, 38, 39, 60])
 @pytest.mark.parametrize("shift", [0.0, 0.25])
-def test_node_values_at_any_scale(exponent, shift):
-    V, F = icosphere(0.5, 3)
+@pytest.mark.parametrize("levels", [2, 3])
+def test_node_values_at_any_scale(exponent, shift, levels):
+    V, F = icosphere(0.5, levels)
     scale = 10.0 ** exponent
     V, lo, hi = (V + shift) * scale, (V.min(0) - 0.25) * scale, (V.max(0) + 0.25) * scale
     print(f"[gpu-case] grid tree at scale 1e{exponent}", flush=True)
