@@ -627,8 +627,9 @@ void build_mesh_grid(hipStream_t s, const double* pos, uint32_t nv, const uint32
         gp.dmin[d] = dmin[d];
     }
     uint64_t const n = grid_dims(res).nodes(), per_block = uint64_t(kRun) * (kBlock / 64);
-    mesh_upload mesh(s, pos, nv, tris, nt);
     dev_buf<uint32_t> nearest_of;
+    if (nt > kScanTriangles) nearest_of.alloc(n);
+    mesh_upload mesh(s, pos, nv, tris, nt);
     if (mesh.view.m <= kScanTriangles) {
         mesh_normals const nm = mesh.normals(s, pos, nv);
         uint32_t const split = n <= kSplitNodes ? 8u : 1u;
@@ -638,7 +639,6 @@ void build_mesh_grid(hipStream_t s, const double* pos, uint32_t nv, const uint32
         hip_check(hipStreamSynchronize(s), "grid node kernel");
         return;
     }
-    nearest_of.alloc(n);
     k_grid_nodes<<<unsigned((n + per_block - 1) / per_block), kBlock, 0, s>>>(mesh.view, gp, n, nearest_of.p);
     hip_check(hipGetLastError(), "grid node kernel");
     mesh_normals const nm = mesh.normals(s, pos, nv);
